@@ -15,7 +15,8 @@ of the guided tracer at equal wall-clock on the door-room scene (1080p, depth
 multi-view batch (64 Cornell variants), `guided_batched` guided plus batched (2 door-room + 2
 terrain variants at 1080p with per-view hash grids and a shared MLP; `--guided-batch-full` runs
 the 16 + 16 views).  The roofline block uses
-the kernel that takes longest alone; its algorithmic bytes come from a counting
+the kernel that takes longest alone (the traversal, which takes a bounce's
+extension rays together with the shadow rays of the bounce before); its algorithmic bytes come from a counting
 pass over the same frames (identical rays: the tracer is deterministic) and its
 time from HIP events recorded during the timed region on the streams of the
 launch's concurrent chains (its active time: the union of its dispatches'
@@ -500,7 +501,7 @@ def summarize_pmc(fetch_dir, write_dir, frames_per_launch, out_path, kernels, ch
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_terrain_1080p.json")
-TRAFFIC_KERNELS = {"trace": "k_trace<false, false>", "shade": "k_shade<false, ", "shadow": "k_shadow<false, false>"}
+TRAFFIC_KERNELS = {"trace": "k_trace<false, false>", "shade": "k_shade<false, "}
 
 
 def measured_traffic(frames_per_launch):
@@ -635,30 +636,33 @@ def main():
         s1 = tracer.stats()
         alone = {k: (s1["ms_" + k] - base1["ms_" + k], s1["launches_" + k] - base1["launches_" + k])
                  for k in ("trace", "shade", "shadow")}
+        log("alone (one chain): " + json.dumps({k: round(v[0], 3) for k, v in alone.items()}))
 
     samples = args.steps * npix
     value = samples / elapsed / 1e6
+    ext_bytes = (rays_ext * (RAY_BYTES + HIT_BYTES) + counted["node_visits"] * NODE_BYTES
+                 + counted["tri_tests"] * TRI_BYTES)
+    shadow_bytes = (rays_shadow * (RAY_BYTES + SHADOW_RESULT_BYTES) + counted["shadow_node_visits"] * NODE_BYTES
+                    + counted["shadow_tri_tests"] * TRI_BYTES)
+    # The timed pass traces a bounce's shadow rays in the launch of the next
+    # bounce's extension rays; the one-chain pass traces them alone.
     kernels = {
-        "trace": (ms["ms_trace"], launches["launches_trace"],
-                  rays_ext * (RAY_BYTES + HIT_BYTES) + counted["node_visits"] * NODE_BYTES
-                  + counted["tri_tests"] * TRI_BYTES),
-        "shadow": (ms["ms_shadow"], launches["launches_shadow"],
-                   rays_shadow * (RAY_BYTES + SHADOW_RESULT_BYTES) + counted["shadow_node_visits"] * NODE_BYTES
-                   + counted["shadow_tri_tests"] * TRI_BYTES),
+        "trace": (ms["ms_trace"], launches["launches_trace"], ext_bytes + shadow_bytes),
         "shade": (ms["ms_shade"], launches["launches_shade"], rays_ext * SHADE_BYTES_PER_VERTEX),
     }
+    alone_bytes = {"trace": ext_bytes, "shadow": shadow_bytes, "shade": kernels["shade"][2]}
     # A launch here is one bounce of the pass (all concurrent chains), and a
     # kernel's time is its active time: the union of its dispatches' intervals
     # (they share the GPU with the other chains' kernels meanwhile).  The
     # one-chain pass gives each kernel's time alone; the dominant kernel is
     # the one that takes longest alone.
-    dominant = max(kernels, key=lambda k: (alone or {k: kernels[k]})[k][0])
+    dominant = max(kernels, key=lambda k: (alone or kernels)[k][0])
     dms, dlaunch, dbytes = kernels[dominant]
     achieved = dbytes / (dms / 1000.0) / 1e9 if dms > 0 else 0.0
     single_chain = None
     if alone:
         ams, alaunch = alone[dominant]
-        achieved_alone = dbytes / (ams / 1000.0) / 1e9 if ams > 0 else 0.0
+        achieved_alone = alone_bytes[dominant] / (ams / 1000.0) / 1e9 if ams > 0 else 0.0
         single_chain = {"avg_launch_ms": round(ams / max(1, alaunch), 4), "achieved": round(achieved_alone, 1),
                         "frac": round(achieved_alone / HBM_PEAK_GBS, 4),
                         "msamples_per_s": round(samples / elapsed1 / 1e6, 3),

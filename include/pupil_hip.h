@@ -224,7 +224,9 @@ typedef struct pt_stats {
     /* Per kernel kind, for launches made with PT_RENDER_TIMING: the time during
      * which at least one of its dispatches ran (HIP events; the kernels of a
      * launch's concurrent chains overlap) and the number of launches timed (a
-     * bounce of all chains counts once). */
+     * bounce of all chains counts once).  A bounce's shadow rays are traced in
+     * the launch of the next bounce's extension rays, which counts as trace;
+     * PT_RENDER_ONE_CHAIN traces them in launches of their own (ms_shadow). */
     double ms_raygen, ms_trace, ms_shade, ms_shadow, ms_accumulate;
     uint64_t launches_trace, launches_shade, launches_shadow;
     uint32_t bvh_nodes, bvh_leaf_tris, bvh_depth;

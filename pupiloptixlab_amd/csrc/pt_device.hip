@@ -3,8 +3,9 @@
 //
 // One frame (= one sample per pixel, as one optixLaunch of the reference,
 // example/path_tracer/pt_pass.cpp:39-57) runs as:
-//   raygen -> { trace -> shade -> shadow } x max_depth -> accumulate
-// over structure-of-arrays path queues.  `spp_per_launch` frames run in the
+//   raygen -> trace -> { shade -> trace } x (max_depth - 1) -> shade -> accumulate
+// over structure-of-arrays path queues; a traversal launch takes the extension
+// rays of a bounce and the shadow rays of the bounce before.  `spp_per_launch` frames run in the
 // same queues concurrently; accumulation then folds them in frame order, so
 // the result equals frame-by-frame rendering bit for bit.
 #include <hip/hip_runtime.h>
@@ -198,107 +199,119 @@ __device__ __forceinline__ uint32_t wave_fetch(uint32_t *work, uint32_t n) {
     return __shfl(base, 0);
 }
 
-// Work distribution of the persistent traversal kernels, 64 items per wave
-// at a time: a wave's first chunk is fixed by its index, later chunks come
-// from the shared cursor (which starts at zero) past the statically assigned
-// range.  When the queue is shorter than the grid, idle waves exit without
-// touching the cursor: one cursor atomic per wave would serialize the whole
-// grid on one address even when there is nothing to trace.
+// Work distribution of the persistent traversal kernel, one chunk of 64 rays
+// per wave at a time: a wave's first chunk is fixed by its index, later
+// chunks come from the shared cursor (which starts at zero) past the
+// statically assigned ones.  When the queues are shorter than the grid, idle
+// waves exit without touching the cursor: one cursor atomic per wave would
+// serialize the whole grid on one address even when there is nothing to
+// trace.
 struct WaveWork {
-    uint32_t base, dyn0;
+    uint32_t chunk, dyn0;
     __device__ __forceinline__ WaveWork() {
         const uint32_t wpb = blockDim.x >> 6;
-        base = (blockIdx.x * wpb + (threadIdx.x >> 6)) * 64u;
-        dyn0 = gridDim.x * wpb * 64u;
+        chunk = blockIdx.x * wpb + (threadIdx.x >> 6);
+        dyn0 = gridDim.x * wpb;
     }
-    __device__ __forceinline__ void next(uint32_t *work) { base = dyn0 + wave_fetch(work, 64u); }
+    __device__ __forceinline__ void next(uint32_t *work) { chunk = dyn0 + wave_fetch(work, 1u); }
 };
 
-// --- closest-hit traversal ------------------------------------------------------
-// Persistent grid sized to the resident occupancy; each wave pulls 64 rays at
-// a time, so waves that drew short traversals keep working.
-// Several scenes can share the queues (batched views): the view of a path
-// sits above bit `path_bits` of its id and selects its tree's root in `roots`
-// (null for a single scene, where path_bits is 31).
-// Five waves per SIMD (at most 96 VGPRs): the closest-hit traversal keeps the
-// next node's load in flight while it tests a leaf's triangles.
+// --- traversal -------------------------------------------------------------------
+// The rays of one launch of k_trace: the extension rays of a bounce, the
+// shadow rays of the bounce before it, or both.  A null count leaves that
+// queue out.  Several scenes can share the queues (batched views): the view of
+// a path sits above bit `path_bits` of its id and selects its tree's root in
+// `roots` (null for a single scene, where path_bits is 31).
+struct TraceJob {
+    PathQueue q;                // extension rays (ray0, ray1 -> hit); shadow rays add to its tl / lr
+    const uint32_t *ext_count;
+    ShadowQueue sq;
+    const uint32_t *shd_count;
+    float4 *out_l;
+    uint32_t *work;             // chunk cursor, zero at launch
+    unsigned long long *stat;   // closest nodes, closest tris, shadow nodes, shadow tris
+    const uint32_t *roots;
+    uint32_t path_bits;
+};
+
+// Closest hits of 64 extension rays.
 template <bool kCount, bool kSph>
-__global__ __launch_bounds__(kTraceBlock, 5) void k_trace(PathQueue q, DeviceBvh bvh, const uint32_t *count_ptr,
-                                                       uint32_t *work, unsigned long long *stat,
-                                                       const uint32_t *roots, uint32_t path_bits) {
-    __shared__ uint2 lds[kLdsStack * kTraceBlock];
-    const uint32_t count = *count_ptr;
-    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
-    TraverseStats st{0, 0};
-    for (WaveWork ww;; ww.next(work)) {
-        const uint32_t base = ww.base;
-        if (base >= count) break;
-        const uint32_t i = base + lane_id();
-        if (i < count) {
-            const float4 r0 = q.ray0[i], r1 = q.ray1[i];
-            const uint32_t root = roots ? roots[f2u(r0.w) >> path_bits] : 0u;
-            Hit h;
-            trace_one<false, kCount, kSph>(bvh, lds + threadIdx.x, gtid, f3of(r0), f3of(r1), kExtTmin,
-                                           kMaxDistance, h, st, root);
-            q.hit[i] = make_float4(h.t, u2f(h.prim), h.b1, h.b2);
-        }
+__device__ __forceinline__ void trace_extension(const TraceJob &j, const DeviceBvh &bvh, uint2 *lds_col, uint32_t gtid,
+                                                uint32_t i, uint32_t count, TraverseStats &st) {
+    if (i >= count) return;
+    const float4 r0 = j.q.ray0[i], r1 = j.q.ray1[i];
+    const uint32_t root = j.roots ? j.roots[f2u(r0.w) >> j.path_bits] : 0u;
+    Hit h;
+    trace_one<false, kCount, kSph>(bvh, lds_col, gtid, f3of(r0), f3of(r1), kExtTmin, kMaxDistance, h, st, root);
+    j.q.hit[i] = make_float4(h.t, u2f(h.prim), h.b1, h.b2);
+}
+
+// 64 shadow rays: an unoccluded one adds its pending contribution to its
+// path.  Targets: bit 31 set = output slot, else slot of the extension queue;
+// the view sits in bits [path_bits, 31), the slot below.
+template <bool kCount, bool kSph>
+__device__ __forceinline__ void trace_shadow(const TraceJob &j, const DeviceBvh &bvh, uint2 *lds_col, uint32_t gtid,
+                                             uint32_t i, uint32_t count, TraverseStats &st) {
+    bool occluded = true;
+    float4 s1 = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < count) {
+        const float4 s0 = j.sq.s0[i];
+        s1 = j.sq.s1[i];
+        const uint32_t root = j.roots ? j.roots[(f2u(s1.w) & 0x7FFFFFFFu) >> j.path_bits] : 0u;
+        Hit h;
+        occluded = trace_one<true, kCount, kSph>(bvh, lds_col, gtid, f3of(s0), f3of(s1), kShadowEps, s0.w, h, st, root);
     }
-    if (kCount) {
-        atomicAdd(stat + 0, (unsigned long long)st.nodes);
-        atomicAdd(stat + 1, (unsigned long long)st.tris);
+    if (!occluded) {
+        const float4 c = j.sq.s2[i];
+        const uint32_t target = f2u(s1.w);
+        const uint32_t slot = target & ((1u << j.path_bits) - 1u);
+        if (target & 0x80000000u) {
+            float4 l = j.out_l[slot];
+            l.x = l.x + c.x;
+            l.y = l.y + c.y;
+            l.z = l.z + c.z;
+            j.out_l[slot] = l;
+        } else {
+            float4 tl = j.q.tl[slot], lr = j.q.lr[slot];
+            tl.w = tl.w + c.x;
+            lr.x = lr.x + c.y;
+            lr.y = lr.y + c.z;
+            j.q.tl[slot] = tl;
+            j.q.lr[slot] = lr;
+        }
     }
 }
 
-// --- shadow (any-hit) traversal ----------------------------------------------------
-// Shadow-ray targets: bit 31 set = output slot, else next-queue slot; the
-// view sits in bits [path_bits, 31), the slot below.
+// Persistent grid sized to the resident occupancy; each wave pulls 64 rays at
+// a time, so waves that drew short traversals keep working.  A bounce's
+// shadow rays go into the launch of the next bounce's extension rays (their
+// results are read only by the shading after it): the tail of one kind of
+// ray, a few long traversals on an otherwise idle chip, is filled by the
+// other kind, and a bounce drains the chip twice instead of three times
+// (against separate launches, image read back: Cornell 60 K triangles 320x180
+// one frame 1.87 -> 1.25 ms, terrain 0.85 M triangles 1080p one frame 8.77 ->
+// 6.89 ms, 2.4 M triangles 1080p 64 frames 117.1 -> 114.7 ms).
+// Five waves per SIMD (at most 96 VGPRs): the closest-hit traversal keeps the
+// next node's load in flight while it tests a leaf's triangles.
 template <bool kCount, bool kSph>
-__global__ __launch_bounds__(kTraceBlock) void k_shadow(ShadowQueue sq, DeviceBvh bvh, const uint32_t *count_ptr,
-                                                        uint32_t *work, PathQueue next, float4 *out_l,
-                                                        unsigned long long *stat, const uint32_t *roots,
-                                                        uint32_t path_bits) {
+__global__ __launch_bounds__(kTraceBlock, 5) void k_trace(TraceJob j, DeviceBvh bvh) {
     __shared__ uint2 lds[kLdsStack * kTraceBlock];
-    const uint32_t count = *count_ptr;
+    const uint32_t ne = j.ext_count ? *j.ext_count : 0u, ns = j.shd_count ? *j.shd_count : 0u;
+    const uint32_t ce = (ne + 63u) >> 6, chunks = ce + ((ns + 63u) >> 6);
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
-    TraverseStats st{0, 0};
-    for (WaveWork ww;; ww.next(work)) {
-        const uint32_t base = ww.base;
-        if (base >= count) break;
-        const uint32_t i = base + lane_id();
-        bool occluded = true;
-        float4 s1 = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (i < count) {
-            const float4 s0 = sq.s0[i];
-            s1 = sq.s1[i];
-            const uint32_t root = roots ? roots[(f2u(s1.w) & 0x7FFFFFFFu) >> path_bits] : 0u;
-            Hit h;
-            occluded = trace_one<true, kCount, kSph>(bvh, lds + threadIdx.x, gtid, f3of(s0), f3of(s1), kShadowEps,
-                                                     s0.w, h, st, root);
-        }
-        if (!occluded) {
-            const float4 c = sq.s2[i];
-            const uint32_t target = f2u(s1.w);
-            const uint32_t slot = target & ((1u << path_bits) - 1u);
-            if (target & 0x80000000u) {
-                const uint32_t p = slot;
-                float4 l = out_l[p];
-                l.x = l.x + c.x;
-                l.y = l.y + c.y;
-                l.z = l.z + c.z;
-                out_l[p] = l;
-            } else {
-                float4 tl = next.tl[slot], lr = next.lr[slot];
-                tl.w = tl.w + c.x;
-                lr.x = lr.x + c.y;
-                lr.y = lr.y + c.z;
-                next.tl[slot] = tl;
-                next.lr[slot] = lr;
-            }
-        }
+    TraverseStats ste{0, 0}, sts{0, 0};
+    for (WaveWork ww;; ww.next(j.work)) {
+        if (ww.chunk >= chunks) break;
+        if (ww.chunk < ce)
+            trace_extension<kCount, kSph>(j, bvh, lds + threadIdx.x, gtid, ww.chunk * 64u + lane_id(), ne, ste);
+        else
+            trace_shadow<kCount, kSph>(j, bvh, lds + threadIdx.x, gtid, (ww.chunk - ce) * 64u + lane_id(), ns, sts);
     }
     if (kCount) {
-        atomicAdd(stat + 0, (unsigned long long)st.nodes);
-        atomicAdd(stat + 1, (unsigned long long)st.tris);
+        atomicAdd(j.stat + 0, (unsigned long long)ste.nodes);
+        atomicAdd(j.stat + 1, (unsigned long long)ste.tris);
+        atomicAdd(j.stat + 2, (unsigned long long)sts.nodes);
+        atomicAdd(j.stat + 3, (unsigned long long)sts.tris);
     }
 }
 
@@ -915,18 +928,11 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_rays(const float *rays, u
 // Traversal variants: counting on/off x sphere leaves present/absent (a
 // triangle-only tree runs without the sphere test, like an OptiX pipeline
 // built without the sphere primitive flag, optix/pipeline.cpp:14-28).
-using TraceKernel = void (*)(PathQueue, DeviceBvh, const uint32_t *, uint32_t *, unsigned long long *,
-                             const uint32_t *, uint32_t);
-using ShadowKernel = void (*)(ShadowQueue, DeviceBvh, const uint32_t *, uint32_t *, PathQueue, float4 *,
-                              unsigned long long *, const uint32_t *, uint32_t);
+using TraceKernel = void (*)(TraceJob, DeviceBvh);
 using TraceRaysKernel = void (*)(const float *, uint32_t, DeviceBvh, uint4 *);
 TraceKernel trace_kernel(bool count, bool sph) {
     return count ? (sph ? k_trace<true, true> : k_trace<true, false>)
                  : (sph ? k_trace<false, true> : k_trace<false, false>);
-}
-ShadowKernel shadow_kernel(bool count, bool sph) {
-    return count ? (sph ? k_shadow<true, true> : k_shadow<true, false>)
-                 : (sph ? k_shadow<false, true> : k_shadow<false, false>);
 }
 using ShadeKernel = void (*)(SceneView, ShadeParams, PathQueue, const uint32_t *, PathQueue, uint32_t *, ShadowQueue,
                             uint32_t *, float4 *, AovBuffers, const BatchViewDev *, uint32_t);
@@ -1132,12 +1138,10 @@ struct pt_ctx {
     std::vector<hipEvent_t> dep_events;
     std::string error;
     int num_cu = 256;
-    uint32_t trace_blocks_per_cu = 8;       // resident closest-hit traversal blocks per CU, sphere variant
+    uint32_t trace_blocks_per_cu = 8;       // resident traversal blocks per CU, sphere variant
     uint32_t trace_blocks_per_cu_tri = 8;   // triangle-only variant
     uint32_t shade_blocks_per_cu = 8;       // resident k_shade<false> blocks (256 threads) per CU
     uint32_t shade_guided_blocks_per_cu = 2;  // resident k_shade_guided<false> blocks per CU
-    uint32_t shadow_blocks_per_cu = 8;      // resident any-hit (shadow) traversal blocks per CU, spheres
-    uint32_t shadow_blocks_per_cu_tri = 8;  // triangle-only variant
 
     // scene (host copies kept for the BVH build)
     bool has_scene = false;
@@ -1427,9 +1431,6 @@ int ensure_queues(pt_ctx *ctx, uint32_t paths, uint32_t max_depth) {
 uint32_t trace_grid(pt_ctx *ctx) {
     return (uint32_t)ctx->num_cu * (ctx->num_spheres > 0 ? ctx->trace_blocks_per_cu : ctx->trace_blocks_per_cu_tri);
 }
-uint32_t shadow_grid(pt_ctx *ctx, bool spheres) {
-    return (uint32_t)ctx->num_cu * (spheres ? ctx->shadow_blocks_per_cu : ctx->shadow_blocks_per_cu_tri);
-}
 // Shading grids.  k_shade<false>: kShadeRounds times the blocks that can be
 // resident at once.  Every block strides over the queue; with many more
 // blocks than slots the dispatcher balances uneven shading work across CUs,
@@ -1445,10 +1446,7 @@ uint32_t shade_grid(pt_ctx *ctx, bool guided, bool training) {
 
 int ensure_spill(pt_ctx *ctx) {
     const uint32_t threads =
-        (uint32_t)ctx->num_cu *
-        std::max(std::max(ctx->trace_blocks_per_cu, ctx->trace_blocks_per_cu_tri),
-                 std::max(ctx->shadow_blocks_per_cu, ctx->shadow_blocks_per_cu_tri)) *
-        kTraceBlock;
+        (uint32_t)ctx->num_cu * std::max(ctx->trace_blocks_per_cu, ctx->trace_blocks_per_cu_tri) * kTraceBlock;
     if (ctx->d_spill && ctx->spill_threads >= threads) return PT_OK;
     dfree(ctx->d_spill);
     // Four areas: one per chain of a launch.
@@ -2250,6 +2248,17 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
     for (uint32_t c = 0; c < nchain; ++c)
         hipLaunchKernelGGL(k_raygen_batch, dim3((uint32_t)ctx->num_cu * 32u), dim3(256), 0, ch[c].stream, ch[c].q[0],
                            b.d_launch, b.d_views, path_bits, ch[c].counters, ctx->num_counters, c, nchain);
+    // The traversal of bounce bb's extension rays, with the shadow rays of the
+    // bounce before it.
+    const TraceKernel tk = trace_kernel(false, !b.spheres.empty());
+    auto trace = [&](const Chain &k, uint32_t bb, bool shadow) {
+        EventTimer t(ctx, timing, k.stream, launch_group ? (launch_group | (bb + 1)) : 0u);
+        const TraceJob job{k.q[bb & 1], k.ext + bb, k.sq, shadow ? k.shd + bb - 1 : nullptr, ctx->d_out_l,
+                           k.twork + bb, ctx->d_stat, b.d_roots, path_bits};
+        hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, k.stream, job, k.bvh);
+        t.stop(kKindTrace);
+    };
+    for (uint32_t c = 0; c < nchain; ++c) trace(ch[c], 0, false);
     int cur = 0;
     for (uint32_t bb = 0; bb < max_depth; ++bb) {
         const int nxt = cur ^ 1;
@@ -2257,13 +2266,6 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
         const bool infer_here = bg.infer && bb < bg.gdepth && bb + 1 < max_depth;
         for (uint32_t c = 0; c < nchain; ++c) {
             const Chain &k = ch[c];
-            {
-                EventTimer t(ctx, timing, k.stream, group);
-                hipLaunchKernelGGL(trace_kernel(false, !b.spheres.empty()), dim3(tg), dim3(kTraceBlock), 0, k.stream,
-                                   k.q[cur], k.bvh, k.ext + bb, k.twork + bb, ctx->d_stat, (const uint32_t *)b.d_roots,
-                                   path_bits);
-                t.stop(kKindTrace);
-            }
             if (bg.infer || bg.train) {
                 GuideShadeArgs ga = k.ga;
                 ga.gout = infer_here ? k.gout : nullptr;
@@ -2287,13 +2289,7 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
                                    (const BatchViewDev *)b.d_views, path_bits);
                 t.stop(kKindShade);
             }
-            {
-                EventTimer t(ctx, timing, k.stream, group);
-                hipLaunchKernelGGL(shadow_kernel(false, !b.spheres.empty()), dim3(shadow_grid(ctx, !b.spheres.empty())),
-                                   dim3(kTraceBlock), 0, k.stream, k.sq, k.bvh, k.shd + bb, k.swork + bb, k.q[nxt],
-                                   ctx->d_out_l, ctx->d_stat + 2, (const uint32_t *)b.d_roots, path_bits);
-                t.stop(kKindShadow);
-            }
+            if (bb + 1 < max_depth) trace(k, bb + 1, true);
         }
         cur = nxt;
     }
@@ -2701,8 +2697,6 @@ int pt_create(int hip_device, pt_ctx **out) {
         };
         resident(reinterpret_cast<const void *>(k_trace<false, true>), ctx->trace_blocks_per_cu);
         resident(reinterpret_cast<const void *>(k_trace<false, false>), ctx->trace_blocks_per_cu_tri);
-        resident(reinterpret_cast<const void *>(k_shadow<false, true>), ctx->shadow_blocks_per_cu);
-        resident(reinterpret_cast<const void *>(k_shadow<false, false>), ctx->shadow_blocks_per_cu_tri);
         int c = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, k_guide_infer, kInferBlock, 0) == hipSuccess && c > 0)
             ctx->infer_blocks_per_cu = (uint32_t)c;
@@ -3376,6 +3370,27 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
                                ctx->height, k.frames, seed, k.counters, ctx->num_counters, k.frame0, k.pix0, k.pixels);
             t.stop(kKindRaygen);
         }
+        // The traversal of bounce b's extension rays together with the shadow
+        // rays of the bounce before it (the last bounce casts none), or in
+        // launches of their own when kernels are to be timed alone.
+        const TraceKernel tk = trace_kernel(ctx->counting, ctx->num_spheres > 0);
+        auto trace = [&](const Chain &k, uint32_t b, bool shadow) {
+            TraceJob job{k.q[b & 1], k.ext + b, k.sq, shadow ? k.shd + b - 1 : nullptr, ctx->d_out_l, k.twork + b,
+                         ctx->d_stat, nullptr, 31u};
+            if (shadow && (p->flags & PT_RENDER_ONE_CHAIN)) {
+                TraceJob sj = job;
+                sj.ext_count = nullptr;
+                sj.work = k.swork + b - 1;
+                EventTimer t(ctx, timing, k.stream, launch_group | b);
+                hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, k.stream, sj, k.bvh);
+                t.stop(kKindShadow);
+                job.shd_count = nullptr;
+            }
+            EventTimer t(ctx, timing, k.stream, launch_group | (b + 1));
+            hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, k.stream, job, k.bvh);
+            t.stop(kKindTrace);
+        };
+        for (uint32_t c = 0; c < nchain; ++c) trace(ch[c], 0, false);
         int cur = 0;
         for (uint32_t b = 0; b < max_depth; ++b) {
             const int nxt = cur ^ 1;
@@ -3385,13 +3400,6 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
             const uint64_t group = launch_group | (b + 1);
             for (uint32_t c = 0; c < nchain; ++c) {
                 const Chain &k = ch[c];
-                {
-                    EventTimer t(ctx, timing, k.stream, group);
-                    hipLaunchKernelGGL(trace_kernel(ctx->counting, ctx->num_spheres > 0), dim3(tg), dim3(kTraceBlock),
-                                       0, k.stream, k.q[cur], k.bvh, k.ext + b, k.twork + b, ctx->d_stat,
-                                       (const uint32_t *)nullptr, 31u);
-                    t.stop(kKindTrace);
-                }
                 GuideShadeArgs gac = ga;
                 gac.gout = infer_here ? k.gout : nullptr;
                 if (infer_here) {
@@ -3413,14 +3421,7 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
                                            ctx->d_out_l, aov, (const BatchViewDev *)nullptr, 31u);
                     t.stop(kKindShade);
                 }
-                {
-                    EventTimer t(ctx, timing, k.stream, group);
-                    hipLaunchKernelGGL(shadow_kernel(ctx->counting, ctx->num_spheres > 0),
-                                       dim3(shadow_grid(ctx, ctx->num_spheres > 0)), dim3(kTraceBlock), 0, k.stream,
-                                       k.sq, k.bvh, k.shd + b, k.swork + b, k.q[nxt], ctx->d_out_l, ctx->d_stat + 2,
-                                       (const uint32_t *)nullptr, 31u);
-                    t.stop(kKindShadow);
-                }
+                if (b + 1 < max_depth) trace(k, b + 1, true);
             }
             cur = nxt;
         }
@@ -3583,11 +3584,9 @@ int pt_render_noalloc(pt_ctx *ctx, const pt_render_params *p) {
     const uint32_t num_counters = 4 * (max_depth + 2);
     const uint32_t tbpc = std::min(kNoAllocTraceBlocksPerCu, ctx->num_spheres > 0 ? ctx->trace_blocks_per_cu
                                                                                  : ctx->trace_blocks_per_cu_tri);
-    const uint32_t sbpc = std::min(kNoAllocTraceBlocksPerCu, ctx->num_spheres > 0 ? ctx->shadow_blocks_per_cu
-                                                                                 : ctx->shadow_blocks_per_cu_tri);
-    const uint32_t tg = (uint32_t)ctx->num_cu * tbpc, shg = (uint32_t)ctx->num_cu * sbpc;
+    const uint32_t tg = (uint32_t)ctx->num_cu * tbpc;
     NoAllocLayout L;
-    if (!noalloc_layout(base, num_counters, std::max(tg, shg) * kTraceBlock, L) || L.capacity < npix) {
+    if (!noalloc_layout(base, num_counters, tg * kTraceBlock, L) || L.capacity < npix) {
         ctx->error = "pt_render_noalloc: one frame of " + std::to_string(npix) + " paths exceeds the " +
                      std::to_string(kNoAllocScratchBytes >> 20) + " MiB scratch (" + std::to_string(L.capacity) +
                      " paths of 224 bytes)";
@@ -3614,7 +3613,7 @@ int pt_render_noalloc(pt_ctx *ctx, const pt_render_params *p) {
         const uint32_t frames = std::min(per_launch, p->spp - done);
         const uint32_t total = frames * npix;
         uint32_t *ext = L.counters, *shd = L.counters + (max_depth + 2);
-        uint32_t *twork = L.counters + 2 * (max_depth + 2), *swork = L.counters + 3 * (max_depth + 2);
+        uint32_t *twork = L.counters + 2 * (max_depth + 2);
         // k_raygen clears every counter before the first traversal reads them.
         const uint32_t rgrid = std::min<uint32_t>((total + 255) / 256, (uint32_t)ctx->num_cu * 32u);
         hipLaunchKernelGGL(k_raygen, dim3(rgrid), dim3(256), 0, ctx->stream, L.q[0], ctx->camera, ctx->width,
@@ -3629,14 +3628,13 @@ int pt_render_noalloc(pt_ctx *ctx, const pt_render_params *p) {
         int cur = 0;
         for (uint32_t b = 0; b < max_depth; ++b) {
             const int nxt = cur ^ 1;
+            const TraceJob job{L.q[cur], ext + b, L.sq, b ? shd + b - 1 : nullptr, L.out_l, twork + b, ctx->d_stat,
+                               nullptr, 31u};
             hipLaunchKernelGGL(trace_kernel(false, ctx->num_spheres > 0), dim3(tg), dim3(kTraceBlock), 0, ctx->stream,
-                               L.q[cur], bvh, ext + b, twork + b, ctx->d_stat, (const uint32_t *)nullptr, 31u);
+                               job, bvh);
             hipLaunchKernelGGL(shade_kernel(false, ctx->shade_feat), dim3(sg), dim3(256), 0, ctx->stream, sv, sp,
                                L.q[cur], ext + b, L.q[nxt], ext + b + 1, L.sq, shd + b, L.out_l, aov,
                                (const BatchViewDev *)nullptr, 31u);
-            hipLaunchKernelGGL(shadow_kernel(false, ctx->num_spheres > 0), dim3(shg), dim3(kTraceBlock), 0,
-                               ctx->stream, L.sq, bvh, shd + b, swork + b, L.q[nxt], L.out_l, ctx->d_stat + 2,
-                               (const uint32_t *)nullptr, 31u);
             cur = nxt;
         }
         const uint32_t agrid = std::min<uint32_t>((npix + 255) / 256, (uint32_t)ctx->num_cu * 16u);
