@@ -86,21 +86,32 @@ __device__ __forceinline__ void load_node_dev(const WideNode *nodes, uint32_t i,
     q[4] = e;
 }
 
+// Traversal stack of one lane: the first entries in LDS, the rest in its spill
+// area.  The address spaces are spelled out: a pointer chosen between the two
+// would make every push and pop a flat access, which waits for all loads in
+// flight.
 struct LdsStack {
-    uint2 *lds;    // this lane's column: lds[k * stride]
-    uint2 *spill;  // this lane's global overflow area
+    typedef __attribute__((address_space(3))) uint64_t lds_entry;
+    typedef __attribute__((address_space(1))) uint64_t spill_entry;
+    lds_entry *lds;      // this lane's column: lds[k * stride]
+    spill_entry *spill;  // this lane's global overflow area
     uint32_t stride;
     uint32_t sp;
+    __device__ LdsStack(uint2 *l, uint2 *s, uint32_t st)
+        : lds((lds_entry *)l), spill((spill_entry *)s), stride(st), sp(0u) {}
     __device__ void push(uint32_t a, uint32_t b) {
-        if (sp < (uint32_t)kLdsStack) lds[sp * stride] = make_uint2(a, b);
-        else spill[sp - kLdsStack] = make_uint2(a, b);
+        const uint64_t v = (uint64_t)b << 32 | a;
+        if (sp < (uint32_t)kLdsStack) lds[sp * stride] = v;
+        else spill[sp - kLdsStack] = v;
         ++sp;
     }
     __device__ void pop(uint32_t &a, uint32_t &b) {
         --sp;
-        uint2 v = sp < (uint32_t)kLdsStack ? lds[sp * stride] : spill[sp - kLdsStack];
-        a = v.x;
-        b = v.y;
+        uint64_t v;
+        if (sp < (uint32_t)kLdsStack) v = lds[sp * stride];
+        else v = spill[sp - kLdsStack];
+        a = (uint32_t)v;
+        b = (uint32_t)(v >> 32);
     }
     __device__ bool empty() const { return sp == 0; }
 };
@@ -108,7 +119,7 @@ struct LdsStack {
 template <bool kAnyHit, bool kCount, bool kSph>
 __device__ __forceinline__ bool trace_one(const DeviceBvh &bvh, uint2 *lds_col, uint32_t gtid, f3 o, f3 d,
                                           float tmin, float tmax, Hit &h, TraverseStats &st, uint32_t root = 0u) {
-    LdsStack stack{lds_col, bvh.spill + (size_t)gtid * kSpillEntries, (uint32_t)kTraceBlock, 0u};
+    LdsStack stack(lds_col, bvh.spill + (size_t)gtid * kSpillEntries, (uint32_t)kTraceBlock);
     auto ln = [&](uint32_t i, NodeWords &n) { load_node_words(bvh.nodes, i, n); };
     auto lt = [&](uint32_t i, LeafTri &t) {
         const float4 *p = reinterpret_cast<const float4 *>(bvh.tris + i);
