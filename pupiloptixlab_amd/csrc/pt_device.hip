@@ -133,18 +133,53 @@ __device__ __forceinline__ bool trace_one(const DeviceBvh &bvh, uint2 *lds_col, 
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
-// Wave-level stream compaction: one atomic per wave reserves slots for the
-// lanes whose predicate holds; each lane gets base + its rank in the ballot.
-__device__ __forceinline__ uint32_t wave_alloc(bool pred, uint32_t *counter) {
-    const unsigned long long mask = __ballot(pred);
-    if (mask == 0ull) return 0u;
-    const uint32_t lane = lane_id();
-    const int leader = __ffsll((long long)mask) - 1;
-    uint32_t base = 0;
-    if ((int)lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader);
-    const unsigned long long lt = lane == 0 ? 0ull : (mask & ((~0ull) >> (64 - lane)));
-    return base + (uint32_t)__popcll(lt);
+// Queue counters of one chain: for each bounce b the size of its extension
+// queue and that of the shadow queue its traversal launch takes along (the
+// shadow rays of bounce b - 1), side by side so that shading reserves in both
+// with one atomic; then the cursors of the traversal launches.
+__host__ __device__ __forceinline__ uint32_t counter_pair(uint32_t b) { return 2u * b; }
+__host__ __device__ __forceinline__ uint32_t counter_cursor(uint32_t max_depth, uint32_t b) {
+    return 2u * (max_depth + 2u) + b;
+}
+__host__ __device__ __forceinline__ uint32_t counter_shadow_cursor(uint32_t max_depth, uint32_t b) {
+    return 3u * (max_depth + 2u) + b;
+}
+constexpr uint32_t counter_count(uint32_t max_depth) { return 4u * (max_depth + 2u); }
+
+// Block-level stream compaction into the next extension queue and the shadow
+// queue: wave counts meet in LDS, one 64-bit atomic per block reserves slots
+// in both, and each lane gets its rank.  Every shading wave of a launch
+// counts into the same word, which the memory side serves one after another,
+// 4-5 ns each: with an atomic per wave and queue they bound the kernel.  Alone
+// (one chain), 16 bounces: a closed room at 8.3 M paths 19.2 -> 8.7 ms, now
+// bound by its queue traffic (4.2 TB/s), and the terrain at 33 M paths 11.9 ->
+// 5.2 ms, now by VALU issue.  All threads of the block must call it.
+struct QueueSlots {
+    uint32_t ext, shadow;
+};
+constexpr uint32_t kMaxShadeWaves = 4;
+__device__ __forceinline__ QueueSlots block_alloc(bool ext, bool shadow, uint32_t *counts) {
+    __shared__ uint32_t wave_count[kMaxShadeWaves];
+    __shared__ unsigned long long wave_base[kMaxShadeWaves];
+    const unsigned long long me = __ballot(ext), ms = __ballot(shadow);
+    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    if (lane == 0) wave_count[wave] = (uint32_t)__popcll(me) | (uint32_t)__popcll(ms) << 16;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long sum = 0;
+        for (uint32_t w = 0; w < waves; ++w) {
+            wave_base[w] = sum;
+            sum += (unsigned long long)(wave_count[w] >> 16) << 32 | (wave_count[w] & 0xFFFFu);
+        }
+        if (sum) {
+            const unsigned long long base = atomicAdd(reinterpret_cast<unsigned long long *>(counts), sum);
+            for (uint32_t w = 0; w < waves; ++w) wave_base[w] += base;
+        }
+    }
+    __syncthreads();
+    const unsigned long long base = wave_base[wave], below = (1ull << lane) - 1ull;
+    return QueueSlots{(uint32_t)base + (uint32_t)__popcll(me & below),
+                      (uint32_t)(base >> 32) + (uint32_t)__popcll(ms & below)};
 }
 
 __device__ __forceinline__ f3 f3of(float4 v) { return mk3(v.x, v.y, v.z); }
@@ -356,8 +391,8 @@ struct BatchViewDev {
 // RGB textures and no environment map, kFeatAll otherwise.
 template <bool kBatch, uint32_t kFeat>
 __global__ __launch_bounds__(256, kBatch ? 1 : 5) void k_shade(SceneView scene, ShadeParams prm, PathQueue in,
-                                               const uint32_t *count_in, PathQueue out, uint32_t *count_out,
-                                               ShadowQueue sq, uint32_t *count_shadow, float4 *out_l,
+                                               const uint32_t *count_in, PathQueue out, uint32_t *counts_out,
+                                               ShadowQueue sq, float4 *out_l,
                                                AovBuffers aov, const BatchViewDev *views, uint32_t path_bits) {
     const uint32_t count = *count_in;
     const uint32_t stride = gridDim.x * blockDim.x;
@@ -411,8 +446,8 @@ __global__ __launch_bounds__(256, kBatch ? 1 : 5) void k_shade(SceneView scene, 
                 shade_path(scene, prm, ps, prim, h.x, h.z, h.w, so, kFeat, aov_write);
             }
         }
-        const uint32_t j = wave_alloc(valid && so.cont, count_out);
-        const uint32_t k = wave_alloc(valid && so.shadow, count_shadow);
+        const QueueSlots slots = block_alloc(valid && so.cont, valid && so.shadow, counts_out);
+        const uint32_t j = slots.ext, k = slots.shadow;
         if (!valid) continue;
         if (so.cont) {
             out.ray0[j] = make_float4(ps.o.x, ps.o.y, ps.o.z, u2f(packed));
@@ -553,8 +588,8 @@ __global__ __launch_bounds__(kInferBlock) void k_guide_infer(GuideView G, PathQu
 // the values of each launch).
 template <bool kBatch>
 __global__ __launch_bounds__(256) void k_shade_guided(SceneView scene, ShadeParams prm, PathQueue in,
-                                                      const uint32_t *count_in, PathQueue out, uint32_t *count_out,
-                                                      ShadowQueue sq, uint32_t *count_shadow, float4 *out_l,
+                                                      const uint32_t *count_in, PathQueue out, uint32_t *counts_out,
+                                                      ShadowQueue sq, float4 *out_l,
                                                       AovBuffers aov, GuideShadeArgs ga, const BatchViewDev *views,
                                                       uint32_t path_bits, const LaunchDesc *ld) {
     const uint32_t count = *count_in;
@@ -617,8 +652,8 @@ __global__ __launch_bounds__(256) void k_shade_guided(SceneView scene, ShadePara
             if (!(m.c >= 0.f && m.c <= 1.f) || !(m.wsum > 0.f) || !isfinite(m.wsum)) use_guide = false;
         }
         if (scatter) guided_scatter(sv, ps, v, use_guide, m, rs, path, so, view);
-        const uint32_t j = wave_alloc(valid && so.cont, count_out);
-        const uint32_t k = wave_alloc(valid && so.shadow, count_shadow);
+        const QueueSlots slots = block_alloc(valid && so.cont, valid && so.shadow, counts_out);
+        const uint32_t j = slots.ext, k = slots.shadow;
         if (!valid) continue;
         if (so.wrote_aov && aov.albedo) {
             const uint32_t f = path / aov.npix;
@@ -906,8 +941,8 @@ __global__ void k_batch_count(const uint32_t *counters, uint32_t max_depth, unsi
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     unsigned long long e = 0, sh = 0;
     for (uint32_t b = 0; b < max_depth; ++b) {
-        e += counters[b];
-        sh += counters[max_depth + 2 + b];
+        e += counters[counter_pair(b)];
+        sh += counters[counter_pair(b + 1) + 1];
     }
     rays[0] += e;
     rays[1] += sh;
@@ -946,7 +981,7 @@ TraceKernel trace_kernel(bool count, bool sph) {
                  : (sph ? k_trace<false, true> : k_trace<false, false>);
 }
 using ShadeKernel = void (*)(SceneView, ShadeParams, PathQueue, const uint32_t *, PathQueue, uint32_t *, ShadowQueue,
-                            uint32_t *, float4 *, AovBuffers, const BatchViewDev *, uint32_t);
+                            float4 *, AovBuffers, const BatchViewDev *, uint32_t);
 // The shading kernel for a scene using the kFeat* features `feat`.
 ShadeKernel shade_kernel(bool batch, uint32_t feat) {
     if (batch) return feat ? k_shade<true, kFeatAll> : k_shade<true, 0u>;
@@ -1417,7 +1452,7 @@ MaterialRec to_material_rec(const pt_material_desc &m, const pt_bitmap_desc *bit
 }
 
 int ensure_queues(pt_ctx *ctx, uint32_t paths, uint32_t max_depth) {
-    uint32_t need_counters = 4 * (max_depth + 2);
+    const uint32_t need_counters = counter_count(max_depth);
     if (paths <= ctx->capacity && need_counters <= ctx->num_counters) return PT_OK;
     free_queues(ctx);
     const size_t n = paths;
@@ -2232,7 +2267,7 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
     const hipStream_t streams[kMaxChains] = {ctx->stream, ctx->stream2, ctx->stream3, ctx->stream4};
     struct Chain {
         hipStream_t stream;
-        uint32_t *counters, *ext, *shd, *twork, *swork;
+        uint32_t *counters;
         PathQueue q[2];
         ShadowQueue sq;
         DeviceBvh bvh;
@@ -2243,10 +2278,6 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
         Chain &k = ch[c];
         k.stream = streams[c];
         k.counters = ctx->d_counters + (size_t)c * ctx->num_counters;
-        k.ext = k.counters;
-        k.shd = k.counters + (max_depth + 2);
-        k.twork = k.counters + 2 * (max_depth + 2);
-        k.swork = k.counters + 3 * (max_depth + 2);
         k.q[0] = queue_at(ctx->q[0], c * share);
         k.q[1] = queue_at(ctx->q[1], c * share);
         k.sq = shadow_queue_at(ctx->sq, c * share);
@@ -2264,8 +2295,9 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
     const TraceKernel tk = trace_kernel(false, !b.spheres.empty());
     auto trace = [&](const Chain &k, uint32_t bb, bool shadow) {
         EventTimer t(ctx, timing, k.stream, launch_group ? (launch_group | (bb + 1)) : 0u);
-        const TraceJob job{k.q[bb & 1], k.ext + bb, k.sq, shadow ? k.shd + bb - 1 : nullptr, ctx->d_out_l,
-                           k.twork + bb, ctx->d_stat, b.d_roots, path_bits};
+        uint32_t *pair = k.counters + counter_pair(bb);
+        const TraceJob job{k.q[bb & 1], pair, k.sq, shadow ? pair + 1 : nullptr, ctx->d_out_l,
+                           k.counters + counter_cursor(max_depth, bb), ctx->d_stat, b.d_roots, path_bits};
         hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, k.stream, job, k.bvh);
         t.stop(kKindTrace);
     };
@@ -2283,20 +2315,22 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
                 if (infer_here) {
                     EventTimer t(ctx, timing, k.stream, group);
                     hipLaunchKernelGGL(k_guide_infer, dim3(ctx->num_cu * ctx->infer_blocks_per_cu), dim3(kInferBlock),
-                                       0, k.stream, bg.view, k.q[cur], k.ext + bb, reinterpret_cast<uint2 *>(k.gout),
+                                       0, k.stream, bg.view, k.q[cur], k.counters + counter_pair(bb),
+                                       reinterpret_cast<uint2 *>(k.gout),
                                        ctx->d_stat + 4, path_bits, InferScene{sv.tri, sv.shapes, sv.spheres, sv.materials});
                     t.stop(kKindGuideInfer);
                 }
                 EventTimer t(ctx, timing, k.stream, group);
                 hipLaunchKernelGGL(k_shade_guided<true>, dim3((uint32_t)ctx->num_cu * sh.shade_bpc), dim3(256), 0,
-                                   k.stream, sv, sp, k.q[cur], k.ext + bb, k.q[nxt], k.ext + bb + 1, k.sq, k.shd + bb,
-                                   ctx->d_out_l, aov, ga, (const BatchViewDev *)b.d_views, path_bits,
+                                   k.stream, sv, sp, k.q[cur], k.counters + counter_pair(bb), k.q[nxt],
+                                   k.counters + counter_pair(bb + 1), k.sq, ctx->d_out_l, aov, ga, (const BatchViewDev *)b.d_views, path_bits,
                                    (const LaunchDesc *)b.d_launch);
                 t.stop(kKindShade);
             } else {
                 EventTimer t(ctx, timing, k.stream, group);
                 hipLaunchKernelGGL(shade_kernel(true, b.feat), dim3(sg), dim3(sh.shade_block), 0, k.stream, sv, sp,
-                                   k.q[cur], k.ext + bb, k.q[nxt], k.ext + bb + 1, k.sq, k.shd + bb, ctx->d_out_l, aov,
+                                   k.q[cur], k.counters + counter_pair(bb), k.q[nxt],
+                                   k.counters + counter_pair(bb + 1), k.sq, ctx->d_out_l, aov,
                                    (const BatchViewDev *)b.d_views, path_bits);
                 t.stop(kKindShade);
             }
@@ -3342,7 +3376,7 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
             uint32_t frame0, frames, pix0, pixels;  // frames x tile-order pixel places of the launch
             uint32_t slot0, paths;                  // its slots [slot0, slot0 + paths) of the queues
             hipStream_t stream;
-            uint32_t *counters, *ext, *shd, *twork, *swork;
+            uint32_t *counters;
             PathQueue q[2];
             ShadowQueue sq;
             DeviceBvh bvh;
@@ -3358,10 +3392,6 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
             k.paths = part[c].paths;
             k.stream = chain_stream[c];
             k.counters = ctx->d_counters + (size_t)c * ctx->num_counters;
-            k.ext = k.counters;                          // extension queue sizes
-            k.shd = k.counters + (max_depth + 2);        // shadow queue sizes
-            k.twork = k.counters + 2 * (max_depth + 2);  // trace work cursors
-            k.swork = k.counters + 3 * (max_depth + 2);  // shadow work cursors
             k.q[0] = queue_at(ctx->q[0], k.slot0);
             k.q[1] = queue_at(ctx->q[1], k.slot0);
             k.sq = shadow_queue_at(ctx->sq, k.slot0);
@@ -3386,12 +3416,13 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
         // launches of their own when kernels are to be timed alone.
         const TraceKernel tk = trace_kernel(ctx->counting, ctx->num_spheres > 0);
         auto trace = [&](const Chain &k, uint32_t b, bool shadow) {
-            TraceJob job{k.q[b & 1], k.ext + b, k.sq, shadow ? k.shd + b - 1 : nullptr, ctx->d_out_l, k.twork + b,
-                         ctx->d_stat, nullptr, 31u};
+            uint32_t *pair = k.counters + counter_pair(b);
+            TraceJob job{k.q[b & 1], pair, k.sq, shadow ? pair + 1 : nullptr, ctx->d_out_l,
+                         k.counters + counter_cursor(max_depth, b), ctx->d_stat, nullptr, 31u};
             if (shadow && (p->flags & PT_RENDER_ONE_CHAIN)) {
                 TraceJob sj = job;
                 sj.ext_count = nullptr;
-                sj.work = k.swork + b - 1;
+                sj.work = k.counters + counter_shadow_cursor(max_depth, b);
                 EventTimer t(ctx, timing, k.stream, launch_group | b);
                 hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, k.stream, sj, k.bvh);
                 t.stop(kKindShadow);
@@ -3416,7 +3447,8 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
                 if (infer_here) {
                     EventTimer t(ctx, timing, k.stream, group);
                     hipLaunchKernelGGL(k_guide_infer, dim3(ctx->num_cu * ctx->infer_blocks_per_cu), dim3(kInferBlock),
-                                       0, k.stream, gview, k.q[cur], k.ext + b, reinterpret_cast<uint2 *>(k.gout),
+                                       0, k.stream, gview, k.q[cur], k.counters + counter_pair(b),
+                                       reinterpret_cast<uint2 *>(k.gout),
                                        ctx->d_stat + 4, 31u, InferScene{sv.tri, sv.shapes, sv.spheres, sv.materials});
                     t.stop(kKindGuideInfer);
                 }
@@ -3424,12 +3456,14 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
                     EventTimer t(ctx, timing, k.stream, group);
                     if (guided)
                         hipLaunchKernelGGL(k_shade_guided<false>, dim3(sg), dim3(256), 0, k.stream, sv, sp, k.q[cur],
-                                           k.ext + b, k.q[nxt], k.ext + b + 1, k.sq, k.shd + b, ctx->d_out_l, aov, gac,
+                                           k.counters + counter_pair(b), k.q[nxt], k.counters + counter_pair(b + 1),
+                                           k.sq, ctx->d_out_l, aov, gac,
                                            (const BatchViewDev *)nullptr, 31u, (const LaunchDesc *)nullptr);
                     else
                         hipLaunchKernelGGL(shade_kernel(false, ctx->shade_feat), dim3(sg), dim3(256), 0, k.stream, sv,
-                                           sp, k.q[cur], k.ext + b, k.q[nxt], k.ext + b + 1, k.sq, k.shd + b,
-                                           ctx->d_out_l, aov, (const BatchViewDev *)nullptr, 31u);
+                                           sp, k.q[cur], k.counters + counter_pair(b), k.q[nxt],
+                                           k.counters + counter_pair(b + 1), k.sq, ctx->d_out_l, aov,
+                                           (const BatchViewDev *)nullptr, 31u);
                     t.stop(kKindShade);
                 }
                 if (b + 1 < max_depth) trace(k, b + 1, true);
@@ -3483,8 +3517,8 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
         for (uint32_t c = 0; c < chains_per_launch[k]; ++c) {
             const uint32_t *cn = hist.data() + ((size_t)k * kMaxChains + c) * ctx->num_counters;
             for (uint32_t b = 0; b < max_depth; ++b) {
-                ctx->stats.rays_extension += cn[b];
-                ctx->stats.rays_shadow += cn[max_depth + 2 + b];
+                ctx->stats.rays_extension += cn[counter_pair(b)];
+                ctx->stats.rays_shadow += cn[counter_pair(b + 1) + 1];
             }
         }
     if (guide_infer) {
@@ -3592,7 +3626,7 @@ int pt_render_noalloc(pt_ctx *ctx, const pt_render_params *p) {
         ctx->error = "pt_render_noalloc: max_depth above 250";
         return PT_ERR_INVALID_ARG;
     }
-    const uint32_t num_counters = 4 * (max_depth + 2);
+    const uint32_t num_counters = counter_count(max_depth);
     const uint32_t tbpc = std::min(kNoAllocTraceBlocksPerCu, ctx->num_spheres > 0 ? ctx->trace_blocks_per_cu
                                                                                  : ctx->trace_blocks_per_cu_tri);
     const uint32_t tg = (uint32_t)ctx->num_cu * tbpc;
@@ -3623,8 +3657,6 @@ int pt_render_noalloc(pt_ctx *ctx, const pt_render_params *p) {
     while (done < p->spp) {
         const uint32_t frames = std::min(per_launch, p->spp - done);
         const uint32_t total = frames * npix;
-        uint32_t *ext = L.counters, *shd = L.counters + (max_depth + 2);
-        uint32_t *twork = L.counters + 2 * (max_depth + 2);
         // k_raygen clears every counter before the first traversal reads them.
         const uint32_t rgrid = std::min<uint32_t>((total + 255) / 256, (uint32_t)ctx->num_cu * 32u);
         hipLaunchKernelGGL(k_raygen, dim3(rgrid), dim3(256), 0, ctx->stream, L.q[0], ctx->camera, ctx->width,
@@ -3639,12 +3671,13 @@ int pt_render_noalloc(pt_ctx *ctx, const pt_render_params *p) {
         int cur = 0;
         for (uint32_t b = 0; b < max_depth; ++b) {
             const int nxt = cur ^ 1;
-            const TraceJob job{L.q[cur], ext + b, L.sq, b ? shd + b - 1 : nullptr, L.out_l, twork + b, ctx->d_stat,
-                               nullptr, 31u};
+            uint32_t *pair = L.counters + counter_pair(b);
+            const TraceJob job{L.q[cur], pair, L.sq, b ? pair + 1 : nullptr, L.out_l,
+                               L.counters + counter_cursor(max_depth, b), ctx->d_stat, nullptr, 31u};
             hipLaunchKernelGGL(trace_kernel(false, ctx->num_spheres > 0), dim3(tg), dim3(kTraceBlock), 0, ctx->stream,
                                job, bvh);
             hipLaunchKernelGGL(shade_kernel(false, ctx->shade_feat), dim3(sg), dim3(256), 0, ctx->stream, sv, sp,
-                               L.q[cur], ext + b, L.q[nxt], ext + b + 1, L.sq, shd + b, L.out_l, aov,
+                               L.q[cur], pair, L.q[nxt], L.counters + counter_pair(b + 1), L.sq, L.out_l, aov,
                                (const BatchViewDev *)nullptr, 31u);
             cur = nxt;
         }
