@@ -295,72 +295,77 @@ PT_HD void trav_init(TravRay &r, NodeLoad load_node, f3 o, f3 d, float tmin, flo
     if (r.have) load_node(node_index, r.n);
 }
 
+// Box tests of node r.n: the current group becomes its hit internal children,
+// and the hit leaves' primitives come out as bits of t_bits (bit i: primitive
+// t_base + i).
+PT_HD void trav_node(TravRay &r, uint32_t &t_base, uint32_t &t_bits) {
+    const uint32_t *w = r.n.w;
+    const uint32_t imask = w[3] >> 24;
+    const bool neg_x = r.idx < 0.f, neg_y = r.idy < 0.f, neg_z = r.idz < 0.f;  // sign of each slab slope
+    // Slab distances of the quantized child boxes: with a = 2^e / d and
+    // b = (origin - o) / d per axis, plane q is at t = q a + b (one FMA).
+    // Rounding differs from decoding the box first by a few ulps, which
+    // the relative node margin covers; triangle tests stay exact.
+    // The near plane of an axis is the low bound when the slope a is
+    // positive and the high bound otherwise (fma is monotone in q), so
+    // the byte arrays are swapped once per node instead of taking a
+    // min and a max per child (Ylitie et al. 2017); the distances are
+    // the same as min(t0, t1) / max(t0, t1).
+    const float ax = u2f((w[3] & 0xFFu) << 23) * r.idx, bx = (u2f(w[0]) - r.o.x) * r.idx;
+    const float ay = u2f(((w[3] >> 8) & 0xFFu) << 23) * r.idy, by = (u2f(w[1]) - r.o.y) * r.idy;
+    const float az = u2f(((w[3] >> 16) & 0xFFu) << 23) * r.idz, bz = (u2f(w[2]) - r.o.z) * r.idz;
+    uint32_t nqx[2], fqx[2], nqy[2], fqy[2], nqz[2], fqz[2];
+    for (int i = 0; i < 2; ++i) {  // selects, not branches
+        nqx[i] = neg_x ? w[14 + i] : w[8 + i];
+        fqx[i] = neg_x ? w[8 + i] : w[14 + i];
+        nqy[i] = neg_y ? w[16 + i] : w[10 + i];
+        fqy[i] = neg_y ? w[10 + i] : w[16 + i];
+        nqz[i] = neg_z ? w[18 + i] : w[12 + i];
+        fqz[i] = neg_z ? w[12 + i] : w[18 + i];
+    }
+    // A hit internal child sets bit 24 + (slot ^ octant), a hit leaf its
+    // unary triangle count at its offset, so one word carries both.  The
+    // bit index of all slots comes first, four to a word: meta's low five
+    // bits, xor the octant for internal children (the only ones whose
+    // bits 3 and 4 are both set).  Empty slots (meta 0) add no bits
+    // whatever their box test says, so no child branches.  The kernel is
+    // bound by instruction issue (VALU busy 100% at 2.4 M triangles); the
+    // branches and mask updates per child cost more than the few box tests
+    // they skipped.  With the undivided barycentrics and the stack's
+    // address spaces: 64 frames at 1080p 106.4 -> 99.4 ms, one frame after
+    // an edit at 540p 4.97 -> 4.25 ms.
+    uint32_t bits = 0;
+    const uint32_t oct4 = r.oct * 0x01010101u;
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t meta4 = w[6 + i];
+        const uint32_t inner4 = meta4 & (meta4 << 1) & 0x10101010u;
+        const uint32_t pos4 = meta4 ^ (oct4 & ((inner4 >> 1) - (inner4 >> 4)));
+        for (int c = 0; c < 4; ++c) {
+            const int k = 4 * i + c;
+            const float txn = fmaf(qbyte(nqx, k), ax, bx), txf = fmaf(qbyte(fqx, k), ax, bx);
+            const float tyn = fmaf(qbyte(nqy, k), ay, by), tyf = fmaf(qbyte(fqy, k), ay, by);
+            const float tzn = fmaf(qbyte(nqz, k), az, bz), tzf = fmaf(qbyte(fqz, k), az, bz);
+            const float tn = fmaxf(fmaxf(txn, tyn), fmaxf(tzn, r.tmin));
+            const float tf = fminf(fminf(txf, tyf), fminf(tzf, r.tbest));
+            const uint32_t unary = tn <= tf * kNodeMarginRatio ? (meta4 >> (8 * c + 5)) & 7u : 0u;
+            bits |= unary << ((pos4 >> (8 * c)) & 31u);
+        }
+    }
+    r.g_base = w[4];
+    r.g_bits = (bits & 0xFF000000u) | imask;
+    t_base = w[5];
+    t_bits = bits & 0x00FFFFFFu;
+}
+
 // One node of the ray's traversal and its leaf primitives.  Returns whether
 // the ray has more to visit (false also once an any-hit ray has found a hit).
 template <bool kAnyHit, bool kSpheres = true, typename Stack, typename NodeLoad, typename TriLoad>
 PT_HD bool trav_step(TravRay &r, NodeLoad load_node, TriLoad load_tri, Stack &stack, Hit &hit,
                      TraverseStats *stats) {
     if (!r.have) return false;
-    const uint32_t *w = r.n.w;
-    const uint32_t imask = w[3] >> 24;
-    const bool neg_x = r.idx < 0.f, neg_y = r.idy < 0.f, neg_z = r.idz < 0.f;  // sign of each slab slope
+    if (stats) stats->nodes++;
     uint32_t t_base, t_bits;
-    {
-        if (stats) stats->nodes++;
-        // Slab distances of the quantized child boxes: with a = 2^e / d and
-        // b = (origin - o) / d per axis, plane q is at t = q a + b (one FMA).
-        // Rounding differs from decoding the box first by a few ulps, which
-        // the relative node margin covers; triangle tests stay exact.
-        // The near plane of an axis is the low bound when the slope a is
-        // positive and the high bound otherwise (fma is monotone in q), so
-        // the byte arrays are swapped once per node instead of taking a
-        // min and a max per child (Ylitie et al. 2017); the distances are
-        // the same as min(t0, t1) / max(t0, t1).
-        const float ax = u2f((w[3] & 0xFFu) << 23) * r.idx, bx = (u2f(w[0]) - r.o.x) * r.idx;
-        const float ay = u2f(((w[3] >> 8) & 0xFFu) << 23) * r.idy, by = (u2f(w[1]) - r.o.y) * r.idy;
-        const float az = u2f(((w[3] >> 16) & 0xFFu) << 23) * r.idz, bz = (u2f(w[2]) - r.o.z) * r.idz;
-        uint32_t nqx[2], fqx[2], nqy[2], fqy[2], nqz[2], fqz[2];
-        for (int i = 0; i < 2; ++i) {  // selects, not branches
-            nqx[i] = neg_x ? w[14 + i] : w[8 + i];
-            fqx[i] = neg_x ? w[8 + i] : w[14 + i];
-            nqy[i] = neg_y ? w[16 + i] : w[10 + i];
-            fqy[i] = neg_y ? w[10 + i] : w[16 + i];
-            nqz[i] = neg_z ? w[18 + i] : w[12 + i];
-            fqz[i] = neg_z ? w[12 + i] : w[18 + i];
-        }
-        // A hit internal child sets bit 24 + (slot ^ octant), a hit leaf its
-        // unary triangle count at its offset, so one word carries both.  The
-        // bit index of all slots comes first, four to a word: meta's low five
-        // bits, xor the octant for internal children (the only ones whose
-        // bits 3 and 4 are both set).  Empty slots (meta 0) add no bits
-        // whatever their box test says, so no child branches.  The kernel is
-        // bound by instruction issue (VALU busy 100% at 2.4 M triangles); the
-        // branches and mask updates per child cost more than the few box tests
-        // they skipped.  With the undivided barycentrics and the stack's
-        // address spaces: 64 frames at 1080p 106.4 -> 99.4 ms, one frame after
-        // an edit at 540p 4.97 -> 4.25 ms.
-        uint32_t bits = 0;
-        const uint32_t oct4 = r.oct * 0x01010101u;
-        for (int i = 0; i < 2; ++i) {
-            const uint32_t meta4 = w[6 + i];
-            const uint32_t inner4 = meta4 & (meta4 << 1) & 0x10101010u;
-            const uint32_t pos4 = meta4 ^ (oct4 & ((inner4 >> 1) - (inner4 >> 4)));
-            for (int c = 0; c < 4; ++c) {
-                const int k = 4 * i + c;
-                const float txn = fmaf(qbyte(nqx, k), ax, bx), txf = fmaf(qbyte(fqx, k), ax, bx);
-                const float tyn = fmaf(qbyte(nqy, k), ay, by), tyf = fmaf(qbyte(fqy, k), ay, by);
-                const float tzn = fmaf(qbyte(nqz, k), az, bz), tzf = fmaf(qbyte(fqz, k), az, bz);
-                const float tn = fmaxf(fmaxf(txn, tyn), fmaxf(tzn, r.tmin));
-                const float tf = fminf(fminf(txf, tyf), fminf(tzf, r.tbest));
-                const uint32_t unary = tn <= tf * kNodeMarginRatio ? (meta4 >> (8 * c + 5)) & 7u : 0u;
-                bits |= unary << ((pos4 >> (8 * c)) & 31u);
-            }
-        }
-        r.g_base = w[4];
-        r.g_bits = (bits & 0xFF000000u) | imask;
-        t_base = w[5];
-        t_bits = bits & 0x00FFFFFFu;
-    }
+    trav_node(r, t_base, t_bits);
     // Closest-hit rays prefetch the next node; any-hit rays usually stop at
     // their first primitive hit, so for them the load waits (fewer registers).
     uint32_t node_index = 0;

@@ -27,6 +27,7 @@
 #include "pt_batch_plan.h"
 #include "pt_chains.h"
 #include "pt_timing.h"
+#include "pt_trace_stream.h"
 #include "pt_bvh_build.h"
 #include "pt_denoise.h"
 #include "pt_guide_state.h"
@@ -114,6 +115,7 @@ struct LdsStack {
         b = (uint32_t)(v >> 32);
     }
     __device__ bool empty() const { return sp == 0; }
+    __device__ void clear() { sp = 0; }
 };
 
 template <bool kAnyHit, bool kCount, bool kSph>
@@ -238,30 +240,6 @@ __global__ void k_raygen(PathQueue q, CameraRec cam, uint32_t width, uint32_t he
     }
 }
 
-// Wave-level work fetch: lane 0 reserves `n` consecutive items for the wave.
-__device__ __forceinline__ uint32_t wave_fetch(uint32_t *work, uint32_t n) {
-    uint32_t base = 0;
-    if (lane_id() == 0) base = atomicAdd(work, n);
-    return __shfl(base, 0);
-}
-
-// Work distribution of the persistent traversal kernel, one chunk of 64 rays
-// per wave at a time: a wave's first chunk is fixed by its index, later
-// chunks come from the shared cursor (which starts at zero) past the
-// statically assigned ones.  When the queues are shorter than the grid, idle
-// waves exit without touching the cursor: one cursor atomic per wave would
-// serialize the whole grid on one address even when there is nothing to
-// trace.
-struct WaveWork {
-    uint32_t chunk, dyn0;
-    __device__ __forceinline__ WaveWork() {
-        const uint32_t wpb = blockDim.x >> 6;
-        chunk = blockIdx.x * wpb + (threadIdx.x >> 6);
-        dyn0 = gridDim.x * wpb;
-    }
-    __device__ __forceinline__ void next(uint32_t *work) { chunk = dyn0 + wave_fetch(work, 1u); }
-};
-
 // --- traversal -------------------------------------------------------------------
 // The rays of one launch of k_trace: the extension rays of a bounce, the
 // shadow rays of the bounce before it, or both.  A null count leaves that
@@ -280,56 +258,29 @@ struct TraceJob {
     uint32_t path_bits;
 };
 
-// Closest hits of 64 extension rays.
-template <bool kCount, bool kSph>
-__device__ __forceinline__ void trace_extension(const TraceJob &j, const DeviceBvh &bvh, uint2 *lds_col, uint32_t gtid,
-                                                uint32_t i, uint32_t count, TraverseStats &st) {
-    if (i >= count) return;
-    const float4 r0 = j.q.ray0[i], r1 = j.q.ray1[i];
-    const uint32_t root = j.roots ? j.roots[f2u(r0.w) >> j.path_bits] : 0u;
-    Hit h;
-    trace_one<false, kCount, kSph>(bvh, lds_col, gtid, f3of(r0), f3of(r1), kExtTmin, kMaxDistance, h, st, root);
-    j.q.hit[i] = make_float4(h.t, u2f(h.prim), h.b1, h.b2);
-}
-
-// 64 shadow rays: an unoccluded one adds its pending contribution to its
-// path.  Targets: bit 31 set = output slot, else slot of the extension queue;
-// the view sits in bits [path_bits, 31), the slot below.
-template <bool kCount, bool kSph>
-__device__ __forceinline__ void trace_shadow(const TraceJob &j, const DeviceBvh &bvh, uint2 *lds_col, uint32_t gtid,
-                                             uint32_t i, uint32_t count, TraverseStats &st) {
-    bool occluded = true;
-    float4 s1 = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (i < count) {
-        const float4 s0 = j.sq.s0[i];
-        s1 = j.sq.s1[i];
-        const uint32_t root = j.roots ? j.roots[(f2u(s1.w) & 0x7FFFFFFFu) >> j.path_bits] : 0u;
-        Hit h;
-        occluded = trace_one<true, kCount, kSph>(bvh, lds_col, gtid, f3of(s0), f3of(s1), kShadowEps, s0.w, h, st, root);
-    }
-    if (!occluded) {
-        const float4 c = j.sq.s2[i];
-        const uint32_t target = f2u(s1.w);
-        const uint32_t slot = target & ((1u << j.path_bits) - 1u);
-        if (target & 0x80000000u) {
-            float4 l = j.out_l[slot];
-            l.x = l.x + c.x;
-            l.y = l.y + c.y;
-            l.z = l.z + c.z;
-            j.out_l[slot] = l;
-        } else {
-            float4 tl = j.q.tl[slot], lr = j.q.lr[slot];
-            tl.w = tl.w + c.x;
-            lr.x = lr.x + c.y;
-            lr.y = lr.y + c.z;
-            j.q.tl[slot] = tl;
-            j.q.lr[slot] = lr;
-        }
+// Adds an unoccluded shadow ray's contribution to its path.  Targets: bit 31
+// set = output slot, else slot of the extension queue; the view sits in bits
+// [path_bits, 31), the slot below.
+__device__ __forceinline__ void add_contribution(const TraceJob &j, uint32_t i) {
+    const float4 c = j.sq.s2[i];
+    const uint32_t target = f2u(j.sq.s1[i].w), slot = target & ((1u << j.path_bits) - 1u);
+    if (target & 0x80000000u) {
+        float4 l = j.out_l[slot];
+        l.x = l.x + c.x;
+        l.y = l.y + c.y;
+        l.z = l.z + c.z;
+        j.out_l[slot] = l;
+    } else {
+        float4 tl = j.q.tl[slot], lr = j.q.lr[slot];
+        tl.w = tl.w + c.x;
+        lr.x = lr.x + c.y;
+        lr.y = lr.y + c.z;
+        j.q.tl[slot] = tl;
+        j.q.lr[slot] = lr;
     }
 }
 
-// Persistent grid sized to the resident occupancy; each wave pulls 64 rays at
-// a time, so waves that drew short traversals keep working.  A bounce's
+// Persistent grid sized to the resident occupancy (trace_stream).  A bounce's
 // shadow rays go into the launch of the next bounce's extension rays (their
 // results are read only by the shading after it): the tail of one kind of
 // ray, a few long traversals on an otherwise idle chip, is filled by the
@@ -337,22 +288,36 @@ __device__ __forceinline__ void trace_shadow(const TraceJob &j, const DeviceBvh 
 // (against separate launches, image read back: Cornell 60 K triangles 320x180
 // one frame 1.87 -> 1.25 ms, terrain 0.85 M triangles 1080p one frame 8.77 ->
 // 6.89 ms, 2.4 M triangles 1080p 64 frames 117.1 -> 114.7 ms).
-// Five waves per SIMD (at most 96 VGPRs): the closest-hit traversal keeps the
-// next node's load in flight while it tests a leaf's triangles.
+// Six waves per SIMD for triangles, five with the sphere test: registers and
+// the 12.5 KB of LDS per block allow as many.
 template <bool kCount, bool kSph>
-__global__ __launch_bounds__(kTraceBlock, 5) void k_trace(TraceJob j, DeviceBvh bvh) {
-    __shared__ uint2 lds[kLdsStack * kTraceBlock];
+__global__ __launch_bounds__(kTraceBlock, kSph ? 5 : 6) void k_trace(TraceJob j, DeviceBvh bvh) {
+    __shared__ StreamLds<kLdsStack> lds[kTraceBlock / 64];
     const uint32_t ne = j.ext_count ? *j.ext_count : 0u, ns = j.shd_count ? *j.shd_count : 0u;
-    const uint32_t ce = (ne + 63u) >> 6, chunks = ce + ((ns + 63u) >> 6);
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     TraverseStats ste{0, 0}, sts{0, 0};
-    for (WaveWork ww;; ww.next(j.work)) {
-        if (ww.chunk >= chunks) break;
-        if (ww.chunk < ce)
-            trace_extension<kCount, kSph>(j, bvh, lds + threadIdx.x, gtid, ww.chunk * 64u + lane_id(), ne, ste);
-        else
-            trace_shadow<kCount, kSph>(j, bvh, lds + threadIdx.x, gtid, (ww.chunk - ce) * 64u + lane_id(), ns, sts);
-    }
+    const uint32_t total = ne + ns, waves = gridDim.x * (kTraceBlock / 64);
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid >> 6));
+    // Chunks of a quarter of a wave's even share, 64 to 256 rays: the cursor is
+    // one word for the whole grid.
+    const uint32_t chunk = min(max(total / (waves * 4u), 64u), 256u);
+    StreamLds<kLdsStack> &L = lds[__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))];
+    LdsStack stack(reinterpret_cast<uint2 *>(&L.stack[0][lane_id()]), bvh.spill + (size_t)gtid * kSpillEntries, 64u);
+    auto load_node = [&](uint32_t i, NodeWords &n) { load_node_words(bvh.nodes, i, n); };
+    auto fetch = [&](uint32_t i, f3 &o, f3 &d, float &tmax, uint32_t &root, bool &any_hit) {
+        any_hit = i >= ne;
+        const float4 a = any_hit ? j.sq.s0[i - ne] : j.q.ray0[i], b = any_hit ? j.sq.s1[i - ne] : j.q.ray1[i];
+        o = f3of(a);
+        d = f3of(b);
+        tmax = any_hit ? a.w : kMaxDistance;
+        root = j.roots ? j.roots[(any_hit ? f2u(b.w) & 0x7FFFFFFFu : f2u(a.w)) >> j.path_bits] : 0u;
+    };
+    auto finish = [&](uint32_t i, bool any_hit, const Hit &h) {
+        if (!any_hit) j.q.hit[i] = make_float4(h.t, u2f(h.prim), h.b1, h.b2);
+        else if (h.prim == kMissPrim) add_contribution(j, i - ne);
+    };
+    trace_stream<kCount, kSph>(L, stack, bvh.tris, load_node, total, chunk, wave, waves, j.work, kExtTmin,
+                               kShadowEps, fetch, finish, ste, sts);
     if (kCount) {
         atomicAdd(j.stat + 0, (unsigned long long)ste.nodes);
         atomicAdd(j.stat + 1, (unsigned long long)ste.tris);

@@ -1,0 +1,81 @@
+"""The persistent traversal at its edges: ray counts around a wave, a chunk and
+a block, trees whose nodes hit many primitives at once for every lane (the
+ring of waiting ray/primitive pairs fills several times per step), coincident
+primitives (equal t: the lower id wins), one bounce only, and shadow rays in a
+launch of their own.  Every render must equal the oracle's: the same float
+operations per path, in the same order, so radiance within 1e-3 of every pixel
+(as the other parity tests; 99.99% of pixels bit-identical)."""
+import numpy as np
+import pytest
+
+import oracle
+import pupiloptixlab_amd as pt
+
+pytestmark = pytest.mark.gpu
+
+STACK = """<scene version="3.0.0">
+  <integrator type="path"><integer name="max_depth" value="{depth}"/></integrator>
+  <sensor type="perspective"><float name="fov" value="40"/>
+    <transform name="to_world"><lookat origin="0.1, 0.2, 4" target="0, 0, 0" up="0, 1, 0"/></transform>
+    <film type="hdrfilm"><integer name="width" value="{w}"/><integer name="height" value="{h}"/></film>
+  </sensor>
+  {shapes}
+  <shape type="rectangle"><transform name="to_world"><scale value="0.5"/><translate value="0, 0, 3.5"/></transform>
+    <bsdf type="diffuse"/><emitter type="area"><rgb name="radiance" value="5, 4, 3"/></emitter></shape>
+  <emitter type="constant"><rgb name="radiance" value="0.3"/></emitter>
+</scene>"""
+
+
+def stack_scene(tmp_path, w, h, depth=4, sheets=60, sphere=False):
+    """Sheets one behind the other, every third one coincident with the one before."""
+    shapes = []
+    for k in range(sheets):
+        z = -0.01 * (k - (1 if k % 3 == 2 else 0))
+        shapes.append(f"""<shape type="rectangle"><transform name="to_world"><translate value="0, 0, {z}"/></transform>
+            <bsdf type="twosided"><bsdf type="diffuse"><rgb name="reflectance" value="{0.2 + 0.01 * k}, 0.5, 0.4"/>
+            </bsdf></bsdf></shape>""")
+    if sphere:
+        shapes.append('<shape type="sphere"><transform name="to_world"><scale value="0.4"/></transform>'
+                      '<bsdf type="diffuse"/></shape>')
+    p = tmp_path / "stack.xml"
+    p.write_text(STACK.format(w=w, h=h, depth=depth, shapes="\n".join(shapes)))
+    return pt.HostScene.load_xml(str(p))
+
+
+def check(tracer, scene, spp, **kw):
+    tracer.set_scene(scene)
+    tracer.build_bvh()
+    tracer.render(spp=spp, **kw)
+    got, prim = tracer.read(pt.BUF_ACCUM), tracer.read(pt.BUF_PRIM_ID)
+    ref = oracle.render(scene.desc, spp=spp, **{k: v for k, v in kw.items() if k == "max_depth"})
+    g, r = got[..., :3].astype(np.float64), ref["accum"][..., :3].astype(np.float64)
+    assert np.all(np.abs(g - r) <= 1e-3 * np.abs(r) + 1e-6)
+    assert np.mean(np.all(g == r, axis=-1)) >= 0.9999
+    assert np.array_equal(prim, ref["prim"])
+
+
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (63, 1, 1), (64, 1, 1), (65, 1, 1), (16, 16, 1), (257, 3, 2),
+                                     (96, 80, 3)])
+@pytest.mark.parametrize("one_chain", [False, True])
+def test_many_primitives_per_node_and_ties(tracer, tmp_path, w, h, spp, one_chain):
+    print(f"case: stacked sheets {w}x{h} {spp} spp one_chain={one_chain}", flush=True)
+    check(tracer, stack_scene(tmp_path, w, h), spp, one_chain=one_chain)
+
+
+@pytest.mark.parametrize("depth", [1, 2, 3])
+def test_first_bounces(tracer, tmp_path, depth):
+    print(f"case: stacked sheets with a sphere 70x50 depth {depth}", flush=True)
+    check(tracer, stack_scene(tmp_path, 70, 50, sphere=True), 2, max_depth=depth)
+
+
+def test_more_rays_than_the_grid(tracer):
+    """1.6 M camera rays: waves refill from the cursor; against the same frames one by one."""
+    print("case: terrain 640x512 5 frames, one launch vs one launch per frame", flush=True)
+    scene = pt.HostScene.generate(pt.SCENE_TERRAIN, seed=5, width=640, height=512, grid=96, spheres=24)
+    tracer.set_scene(scene)
+    tracer.build_bvh()
+    tracer.render(spp=5)
+    a = tracer.read(pt.BUF_ACCUM)
+    tracer.reset()
+    tracer.render(spp=5, spp_per_launch=1, one_chain=True)
+    assert np.array_equal(a, tracer.read(pt.BUF_ACCUM))
