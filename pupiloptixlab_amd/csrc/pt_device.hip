@@ -1442,17 +1442,20 @@ int ensure_queues(pt_ctx *ctx, uint32_t paths, uint32_t max_depth) {
 uint32_t trace_grid(pt_ctx *ctx) {
     return (uint32_t)ctx->num_cu * (ctx->num_spheres > 0 ? ctx->trace_blocks_per_cu : ctx->trace_blocks_per_cu_tri);
 }
-// Shading grids.  k_shade<false>: kShadeRounds times the blocks that can be
-// resident at once.  Every block strides over the queue; with many more
-// blocks than slots the dispatcher balances uneven shading work across CUs,
-// and blocks that find no work exit at once.  Terrain 1080p, 64 spp,
-// k_shade<false> per render at 1, 4, 16 and 64 rounds: 49.2, 48.0, 46.9 and
-// 46.3 ms.  k_shade_guided<false> uses the same rounds when it only samples;
+// Shading grid for a chain of `paths` queue slots: a block for every 256 of
+// them, at most kShadeRounds times the blocks that can be resident at once.
+// Every block strides over the queue; with many more blocks than slots the
+// dispatcher balances uneven shading work across CUs, and blocks that find no
+// work exit at once (terrain 1080p, 64 frames, image read back, at 1, 4, 16
+// and 64 rounds: 88.9, 87.2, 86.2 and 85.9 ms).  More blocks than slots only
+// cost their dispatch, 15 us a bounce (Cornell 320x180, one frame: 1.10 ->
+// 1.01 ms).  k_shade_guided<false> uses the same rounds when it only samples;
 // while training it keeps a grid of 8 blocks per CU (its training records are
 // indexed by path and vertex, so the grid does not change them).
-uint32_t shade_grid(pt_ctx *ctx, bool guided, bool training) {
-    if (guided && training) return (uint32_t)ctx->num_cu * 8u;
-    return (uint32_t)ctx->num_cu * kShadeRounds * (guided ? ctx->shade_guided_blocks_per_cu : ctx->shade_blocks_per_cu);
+uint32_t shade_grid(pt_ctx *ctx, bool guided, bool training, uint32_t paths) {
+    const uint32_t need = (paths + 255u) / 256u, cus = (uint32_t)ctx->num_cu;
+    if (guided && training) return std::min(need, cus * 8u);
+    return std::min(need, cus * kShadeRounds * (guided ? ctx->shade_guided_blocks_per_cu : ctx->shade_blocks_per_cu));
 }
 
 int ensure_spill(pt_ctx *ctx) {
@@ -3254,7 +3257,7 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
     sp.rr_depth = p->rr_depth;
     sp.mis_mode = p->mis_mode;
     sp.aov = (p->flags & PT_RENDER_AOV) ? 1u : 0u;
-    const uint32_t tg = trace_grid(ctx), sg = shade_grid(ctx, guided, guide_train);
+    const uint32_t tg = trace_grid(ctx);
 
     const uint32_t batches = (p->spp + per_launch - 1) / per_launch;
     const uint32_t hist_elems = std::max(1u, batches) * 4u * ctx->num_counters;  // one set per chain
@@ -3340,6 +3343,7 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
         struct Chain {
             uint32_t frame0, frames, pix0, pixels;  // frames x tile-order pixel places of the launch
             uint32_t slot0, paths;                  // its slots [slot0, slot0 + paths) of the queues
+            uint32_t shade_grid;
             hipStream_t stream;
             uint32_t *counters;
             PathQueue q[2];
@@ -3355,6 +3359,7 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
             k.pixels = part[c].pixels;
             k.slot0 = part[c].slot0;
             k.paths = part[c].paths;
+            k.shade_grid = shade_grid(ctx, guided, guide_train, k.paths);
             k.stream = chain_stream[c];
             k.counters = ctx->d_counters + (size_t)c * ctx->num_counters;
             k.q[0] = queue_at(ctx->q[0], k.slot0);
@@ -3420,12 +3425,12 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
                 {
                     EventTimer t(ctx, timing, k.stream, group);
                     if (guided)
-                        hipLaunchKernelGGL(k_shade_guided<false>, dim3(sg), dim3(256), 0, k.stream, sv, sp, k.q[cur],
+                        hipLaunchKernelGGL(k_shade_guided<false>, dim3(k.shade_grid), dim3(256), 0, k.stream, sv, sp, k.q[cur],
                                            k.counters + counter_pair(b), k.q[nxt], k.counters + counter_pair(b + 1),
                                            k.sq, ctx->d_out_l, aov, gac,
                                            (const BatchViewDev *)nullptr, 31u, (const LaunchDesc *)nullptr);
                     else
-                        hipLaunchKernelGGL(shade_kernel(false, ctx->shade_feat), dim3(sg), dim3(256), 0, k.stream, sv,
+                        hipLaunchKernelGGL(shade_kernel(false, ctx->shade_feat), dim3(k.shade_grid), dim3(256), 0, k.stream, sv,
                                            sp, k.q[cur], k.counters + counter_pair(b), k.q[nxt],
                                            k.counters + counter_pair(b + 1), k.sq, ctx->d_out_l, aov,
                                            (const BatchViewDev *)nullptr, 31u);
@@ -3617,7 +3622,7 @@ int pt_render_noalloc(pt_ctx *ctx, const pt_render_params *p) {
     sp.rr_depth = p->rr_depth;
     sp.mis_mode = p->mis_mode;
     sp.aov = (p->flags & PT_RENDER_AOV) ? 1u : 0u;
-    const uint32_t sg = shade_grid(ctx, false, false);
+    const uint32_t sg = shade_grid(ctx, false, false, per_launch * npix);
     uint32_t done = 0, sample_cnt = ctx->sample_cnt, seed = ctx->random_seed;
     while (done < p->spp) {
         const uint32_t frames = std::min(per_launch, p->spp - done);
