@@ -183,29 +183,37 @@ PT_HD int frexp_exponent(double x) {
 
 // Quantization of one axis of a wide node: the smallest power-of-two step
 // 2^e (e >= -126) for which 8-bit codes exist whose decode p + q 2^e (in
-// float) contains every child interval [clo, chi].  Returns false when no
-// exponent up to 127 works.  The same rule serves the host builder and the
-// GPU refit.
+// float) contains every child interval [clo, chi].  The same rule serves the
+// host builder and the GPU refit: quantize_first_exponent is where the search
+// starts, quantize_child the codes of one child under one step (false when
+// there are none).
+PT_HD int quantize_first_exponent(float p, float node_hi) {
+    const double extent = (double)node_hi - (double)p;
+    if (!(extent > 0.0)) return -126;
+    const int ex = frexp_exponent(extent / 255.0);
+    return ex > -126 ? ex : -126;
+}
+PT_HD bool quantize_child(float p, int e, float clo, float chi, int &ql, int &qh) {
+    const float sc = u2f((uint32_t)(e + 127) << 23);
+    const double lo = floor(((double)clo - (double)p) / (double)sc);
+    const double hi = ceil(((double)chi - (double)p) / (double)sc);
+    ql = (int)fmax(0.0, fmin(255.0, lo));
+    qh = (int)fmax(0.0, fmin(255.0, hi));
+    while (ql > 0 && !(p + (float)ql * sc <= clo)) --ql;
+    if (!(p + (float)ql * sc <= clo)) return false;
+    while (qh < 255 && !(p + (float)qh * sc >= chi)) ++qh;
+    return p + (float)qh * sc >= chi;
+}
+
+// All children of an axis (host).  Returns false when no exponent up to 127
+// works.
 PT_HD bool quantize_node_axis(float p, float node_hi, const float *clo, const float *chi, int n, uint8_t &e_out,
                               uint8_t *qlo, uint8_t *qhi) {
-    const double extent = (double)node_hi - (double)p;
-    int e = -126;
-    if (extent > 0.0) {
-        const int ex = frexp_exponent(extent / 255.0);
-        e = ex > -126 ? ex : -126;
-    }
-    for (; e <= 127; ++e) {
-        const float sc = u2f((uint32_t)(e + 127) << 23);
+    for (int e = quantize_first_exponent(p, node_hi); e <= 127; ++e) {
         bool ok = true;
         for (int i = 0; i < n && ok; ++i) {
-            const double lo = floor(((double)clo[i] - (double)p) / (double)sc);
-            const double hi = ceil(((double)chi[i] - (double)p) / (double)sc);
-            int ql = (int)fmax(0.0, fmin(255.0, lo));
-            int qh = (int)fmax(0.0, fmin(255.0, hi));
-            while (ql > 0 && !(p + (float)ql * sc <= clo[i])) --ql;
-            if (!(p + (float)ql * sc <= clo[i])) ok = false;
-            while (ok && qh < 255 && !(p + (float)qh * sc >= chi[i])) ++qh;
-            if (ok && !(p + (float)qh * sc >= chi[i])) ok = false;
+            int ql, qh;
+            ok = quantize_child(p, e, clo[i], chi[i], ql, qh);
             if (ok) {
                 qlo[i] = (uint8_t)ql;
                 qhi[i] = (uint8_t)qh;
