@@ -295,26 +295,49 @@ __global__ __launch_bounds__(kTrainBlock) void k_guide_train(GuideView G, const 
                     const float gv = dx[2 * c + (s >> 2)][s & 3];
                     dy[c][s] = (_Float16)((float)act[l][c][s] > 0.f ? gv : 0.f);
                 }
-        } else if (valid) {
-            // Hash-table gradient of this lane's four levels.
+        } else {
+            // Feature gradients of this lane's four levels, for the scatter.
+            wave_sync_lds();
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const float g0 = dx[t >> 1][2 * (t & 1)] * inv_scale;
-                const float g1 = dx[t >> 1][2 * (t & 1) + 1] * inv_scale;
-                if (g0 == 0.f && g1 == 0.f) continue;
+                float g0 = valid ? dx[t >> 1][2 * (t & 1)] * inv_scale : 0.f;
+                float g1 = valid ? dx[t >> 1][2 * (t & 1) + 1] * inv_scale : 0.f;
                 if (!isfinite(g0) || !isfinite(g1)) {
                     bad = true;
-                    continue;
+                    g0 = g1 = 0.f;
                 }
-                const int level = guide_lane_level(g, t);
-                LevelCorners lc;
-                level_corners(G, level, u, lc);
-                float2 *tg = B.table_grad + guide_level_base(G, grid, level);
+                *reinterpret_cast<float2 *>(st + (i * kGuideLevels + guide_lane_level(g, t)) * 2) = make_float2(g0, g1);
+            }
+            wave_sync_lds();
+        }
+    }
+    // Hash-table gradient, four (sample, level) pairs at a time: lane
+    // 16 s + 2 k + f adds feature f of corner k for pair s.  A pair's eight
+    // corners mostly share a brick of the table, so its sixteen atomics fall
+    // into two to four lines; with a level per lane every lane of an atomic
+    // went to a line of its own (465 K samples: 6.93 -> 1.90 ms; 16 K: 242 ->
+    // 81 us, 44 us without any atomics).
+    {
+        const int q = lane >> 4, k = (lane >> 1) & 7, f = lane & 1;
+        f3 us[4];
+        uint32_t gs[4];
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    unsafeAtomicAdd(&tg[lc.idx[k]].x, lc.w[k] * g0);
-                    unsafeAtomicAdd(&tg[lc.idx[k]].y, lc.w[k] * g1);
-                }
+        for (int b = 0; b < 4; ++b) {
+            const int src = 4 * b + q;  // lane of sample 4 b + q in group 0
+            us[b] = mk3(__shfl(u.x, src), __shfl(u.y, src), __shfl(u.z, src));
+            gs[b] = (uint32_t)__shfl((int)grid, src);
+        }
+#pragma unroll 2
+        for (int level = 0; level < kGuideLevels; ++level) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const float gv = st[((4 * b + q) * kGuideLevels + level) * 2 + f];
+                if (gv == 0.f) continue;
+                uint32_t idx;
+                float w;
+                level_corner(G, level, us[b], k, idx, w);
+                unsafeAtomicAdd(reinterpret_cast<float *>(B.table_grad + guide_level_base(G, gs[b], level) + idx) + f,
+                                w * gv);
             }
         }
     }

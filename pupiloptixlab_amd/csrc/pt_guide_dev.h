@@ -89,6 +89,17 @@ __device__ __forceinline__ void level_corners(const GuideView &G, int level, f3 
     }
 }
 
+// Corner k of one level: table index and trilinear weight.
+__device__ __forceinline__ void level_corner(const GuideView &G, int level, f3 u, int k, uint32_t &idx, float &w) {
+    const uint32_t res = G.levels[level].res, dense = G.levels[level].dense;
+    const float x = u.x * (float)res, y = u.y * (float)res, z = u.z * (float)res;
+    const uint32_t cx = min((uint32_t)x, res - 1u), cy = min((uint32_t)y, res - 1u), cz = min((uint32_t)z, res - 1u);
+    const float fx = x - (float)cx, fy = y - (float)cy, fz = z - (float)cz;
+    const uint32_t dx = k & 1, dy = (k >> 1) & 1, dz = (k >> 2) & 1;
+    idx = guide_corner_index(res, dense, G.mask, cx + dx, cy + dy, cz + dz);
+    w = (dx ? fx : 1.f - fx) * (dy ? fy : 1.f - fy) * (dz ? fz : 1.f - fz);
+}
+
 // First-layer B operand of lane group g for the query at normalized position
 // u in hash grid `grid`.
 __device__ __forceinline__ half8 guide_encode(const GuideView &G, f3 u, int g, uint32_t grid = 0u) {
