@@ -50,7 +50,8 @@ __device__ __forceinline__ void wave_sync_lds() {
 // samples are packed at [0, n_samples).
 __global__ void k_guide_begin(GuideCtl *ctl, uint32_t first, uint32_t batch, uint32_t capacity, float fp_explicit,
                               uint32_t all_slots) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    ctl->loss_part[threadIdx.x][0] = ctl->loss_part[threadIdx.x][1] = 0.f;
+    if (threadIdx.x != 0) return;
     const uint32_t n = all_slots ? capacity : min(ctl->n_samples, capacity);
     const uint32_t valid = n > first ? min(batch, n - first) : 0u;
     ctl->batch_valid = valid;
@@ -245,8 +246,9 @@ __global__ __launch_bounds__(kTrainBlock) void k_guide_train(GuideView G, const 
             vc += __shfl_xor(vc, off);
         }
         if (lane == 0 && vc > 0.f) {
-            unsafeAtomicAdd(&ctl->loss_sum, ls);
-            unsafeAtomicAdd(&ctl->loss_cnt, vc);
+            float *part = ctl->loss_part[(base >> 4) % kGuideParts];
+            unsafeAtomicAdd(&part[0], ls);
+            unsafeAtomicAdd(&part[1], vc);
         }
     }
     wave_sync_lds();
@@ -357,6 +359,18 @@ __global__ __launch_bounds__(64) void k_guide_dw(const uint16_t *xt, const uint1
     const uint32_t q1 = min(rows, q0 + kGuideDwSlice);
     const int layer = blockIdx.y;
     const int lane = (int)__lane_id();
+    if (blockIdx.x == 0 && layer == 0) {  // the step's loss and weight total, for the kernels that follow
+        float ls = ctl->loss_part[lane][0], vc = ctl->loss_part[lane][1];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            ls += __shfl_xor(ls, off);
+            vc += __shfl_xor(vc, off);
+        }
+        if (lane == 0) {
+            ctl->loss_sum = ls;
+            ctl->loss_cnt = vc;
+        }
+    }
     const int g = lane >> 4, i = lane & 15;
     const int ktiles = layer == 0 ? 2 : 4;
     floatx4 acc[4][4];
@@ -658,15 +672,23 @@ __global__ __launch_bounds__(256) void k_guide_collect_count(const float4 *out_l
             else ++z;
         }
     }
+    // One atomic per block and counter (an atomic per wave was most of the
+    // kernel: 0.92 M record slots 173 -> 34 us).
+    __shared__ uint32_t sum[2];
+    if (threadIdx.x < 2) sum[threadIdx.x] = 0u;
+    __syncthreads();
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         nz += __shfl_xor(nz, off);
         z += __shfl_xor(z, off);
     }
     if (__lane_id() == 0) {
-        if (nz) atomicAdd(&ctl->n_nonzero, nz);
-        if (z) atomicAdd(&ctl->n_zero, z);
+        atomicAdd(&sum[0], nz);
+        atomicAdd(&sum[1], z);
     }
+    __syncthreads();
+    if (threadIdx.x == 0 && sum[0]) atomicAdd(&ctl->n_nonzero, sum[0]);
+    if (threadIdx.x == 1 && sum[1]) atomicAdd(&ctl->n_zero, sum[1]);
 }
 
 // Turns the completed records of one launch into training samples.  Samples
@@ -994,7 +1016,7 @@ bool GuideState::collect(const float4 *out_l, uint32_t total_paths, const GuideR
     }
     hipLaunchKernelGGL(k_guide_collect_begin, dim3(1), dim3(64), 0, stream, ctl);
     const uint32_t grid = std::max(1u, std::min<uint32_t>((r.capacity + 255) / 256, 4096u));
-    hipLaunchKernelGGL(k_guide_collect_count, dim3(grid), dim3(256), 0, stream, out_l, total_paths, r, ctl);
+    hipLaunchKernelGGL(k_guide_collect_count, dim3(std::min(grid, 2048u)), dim3(256), 0, stream, out_l, total_paths, r, ctl);
     hipLaunchKernelGGL(k_guide_collect, dim3(grid), dim3(256), 0, stream, out_l, total_paths, r, samples, cap, ctl,
                        ring_n);
     if (ring_n)

@@ -23,6 +23,11 @@ constexpr float kGuideScaleMax = 32768.f;
 constexpr uint32_t kGuideScaleGrowth = 1000;  // finite steps before the scale doubles
 constexpr uint32_t kGuideDwSlice = 512;   // samples per weight-gradient partial
 
+// Sums that every wave or block of a kernel adds to are spread over this many
+// cache lines: the memory side serves atomics on one word one after another,
+// 4-5 ns each.
+constexpr uint32_t kGuideParts = 64;
+
 struct GuideCtl {
     float loss_scale;
     uint32_t step;         // applied Adam steps
@@ -44,6 +49,8 @@ struct GuideCtl {
     float fp_norm;         // selection-loss normalization of the current step
     uint32_t ring_head;    // next slot of the sample ring (collections into a ring)
     uint32_t ring_start;   // first slot of the current ring collection
+    float pad[11];
+    float loss_part[kGuideParts][32];  // weighted loss and weight total of the step, in parts (first two words)
 };
 
 // Training records written by the guided shading kernel, one per guided
