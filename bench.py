@@ -18,10 +18,10 @@ the 16 + 16 views).  The roofline block uses
 the kernel that takes longest alone (the traversal, which takes a bounce's
 extension rays together with the shadow rays of the bounce before); its algorithmic bytes come from a counting
 pass over the same frames (identical rays: the tracer is deterministic) and its
-time from HIP events recorded during the timed region on the streams of the
-launch's concurrent chains (its active time: the union of its dispatches'
-intervals); `roofline.single_chain` repeats the frames with every launch as one
-chain and prices the kernel alone.  The CPU baseline is the oracle (scalar C++,
+time from HIP events recorded during the timed region (its active time: the
+union of its dispatches' intervals); `roofline.single_chain` repeats the frames
+with shadow rays traced in launches of their own and prices the extension
+rays' kernel alone.  The CPU baseline is the oracle (scalar C++,
 multithreaded) on a bounded band of rows of the same frame.
 """
 import argparse
@@ -624,8 +624,8 @@ def main():
     rays_shadow = s["rays_shadow"] - base["rays_shadow"]
     assert rays_ext == counted["rays_extension"], "timed and counting passes diverged"
 
-    # The same frames once more (untimed for `value`) with each launch as one
-    # chain of kernels: the dominant kernel's event time when it runs alone.
+    # The same frames once more (untimed for `value`) with shadow rays traced
+    # in launches of their own: the extension rays' event time alone.
     alone, elapsed1 = None, None
     if not args.no_single_chain:
         tracer.reset()
@@ -651,11 +651,9 @@ def main():
         "shade": (ms["ms_shade"], launches["launches_shade"], rays_ext * SHADE_BYTES_PER_VERTEX),
     }
     alone_bytes = {"trace": ext_bytes, "shadow": shadow_bytes, "shade": kernels["shade"][2]}
-    # A launch here is one bounce of the pass (all concurrent chains), and a
-    # kernel's time is its active time: the union of its dispatches' intervals
-    # (they share the GPU with the other chains' kernels meanwhile).  The
-    # one-chain pass gives each kernel's time alone; the dominant kernel is
-    # the one that takes longest alone.
+    # A launch here is one bounce of the pass, and a kernel's time the union of
+    # its dispatches' intervals; the dominant kernel is the one that takes
+    # longest in the one-chain pass.
     dominant = max(kernels, key=lambda k: (alone or kernels)[k][0])
     dms, dlaunch, dbytes = kernels[dominant]
     achieved = dbytes / (dms / 1000.0) / 1e9 if dms > 0 else 0.0
@@ -666,7 +664,7 @@ def main():
         single_chain = {"avg_launch_ms": round(ams / max(1, alaunch), 4), "achieved": round(achieved_alone, 1),
                         "frac": round(achieved_alone / HBM_PEAK_GBS, 4),
                         "msamples_per_s": round(samples / elapsed1 / 1e6, 3),
-                        "pass": "the same frames again with every launch as one chain (not part of value)"}
+                        "pass": "the same frames again with shadow rays in launches of their own (not part of value)"}
     # Frames per launch of the timed render (pt_render's default width: up to
     # 64 frames and 128M paths per launch).
     frames_per_launch = args.spp_per_launch or max(1, min(64, (128 << 20) // npix))
@@ -752,7 +750,7 @@ def main():
             "single_chain": single_chain,
             "algorithmic_bytes_per_launch": int(dbytes / max(1, dlaunch)),
             "avg_launch_ms": round(dms / max(1, dlaunch), 4),
-            "launch": ("one bounce of the pass (all concurrent chains); avg_launch_ms is the kernel's active time "
+            "launch": ("one bounce of the pass; avg_launch_ms is the kernel's active time "
                        "(union of its dispatch intervals) per bounce"),
             "frames_per_launch": frames_per_launch,
             "measured_copy_GBps": round(copy_gbps, 1),

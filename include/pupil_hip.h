@@ -183,11 +183,9 @@ enum pt_render_flags {
     PT_RENDER_GUIDE = 8,      /* sample with the learned guiding proposal (needs
                                  pt_guide_enable and PT_MIS_CONSISTENT) */
     PT_RENDER_GUIDE_TRAIN = 16, /* train the guide online on this render's paths */
-    PT_RENDER_ONE_CHAIN = 32    /* run every launch as one chain of kernels (by default a launch's
-                                   paths are split into up to four chains of at least 10^6 paths,
-                                   run concurrently on streams of their own; the image is the same
-                                   either way, and with one chain each kernel's event time is that
-                                   of the kernel alone) */
+    PT_RENDER_ONE_CHAIN = 32    /* trace shadow rays in launches of their own instead of together
+                                   with the next bounce's extension rays; the image is the same
+                                   either way, and each kind of ray is timed alone */
 };
 
 /* Launch parameters (example/path_tracer/type.h:9-33 config + pass knobs). */
@@ -222,9 +220,8 @@ typedef struct pt_stats {
     uint64_t shadow_tri_tests;
     double ms_total;         /* wall time of pt_render calls */
     /* Per kernel kind, for launches made with PT_RENDER_TIMING: the time during
-     * which at least one of its dispatches ran (HIP events; the kernels of a
-     * launch's concurrent chains overlap) and the number of launches timed (a
-     * bounce of all chains counts once).  A bounce's shadow rays are traced in
+     * which at least one of its dispatches ran (HIP events) and the number of
+     * launches timed (one per bounce).  A bounce's shadow rays are traced in
      * the launch of the next bounce's extension rays, which counts as trace;
      * PT_RENDER_ONE_CHAIN traces them in launches of their own (ms_shadow). */
     double ms_raygen, ms_trace, ms_shade, ms_shadow, ms_accumulate;

@@ -477,8 +477,8 @@ class PathTracer:
                one_chain: bool = False) -> None:
         """Renders `spp` frames.  guide: sample with the learned proposal;
         guide_train: train it on this render's paths (both need
-        guide_enable() and mis_mode=MIS_CONSISTENT); one_chain: run each
-        launch as one chain of kernels (same image)."""
+        guide_enable() and mis_mode=MIS_CONSISTENT); one_chain: trace
+        shadow rays in launches of their own (same image)."""
         flags = (RENDER_AOV if aov else 0) | (RENDER_FP64_ACCUM if fp64 else 0) | (RENDER_TIMING if timing else 0)
         flags |= (RENDER_GUIDE if guide else 0) | (RENDER_GUIDE_TRAIN if guide_train else 0)
         flags |= RENDER_ONE_CHAIN if one_chain else 0

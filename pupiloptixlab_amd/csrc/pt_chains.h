@@ -1,7 +1,6 @@
-// How a launch's paths split into concurrent chains of kernels (pt_render and
-// batched launches), shared by the host code that plans the chains, the
-// raygen kernels that fill each chain's queue part, and the host tests
-// (tests/chain_sim.cpp).
+// How a launch's paths split into chains of kernels: which frame and pixel a
+// queue slot holds (raygen), and the shares of several chains, as planned by
+// hosts that run more than one (tests/chain_sim.cpp; a launch here runs one).
 #pragma once
 
 #include <cstdint>
@@ -16,10 +15,16 @@ namespace pupil {
 
 // At most this many chains per launch, of at least kChainPaths paths each;
 // batched queues hold a multiple of kChainLcm slots, so every chain count
-// divides them.
-constexpr uint32_t kMaxChains = 4;
+// divides them.  One: while a wave waited for its slowest ray and shading for
+// its counters, concurrent chains filled the idle CUs; now a chain keeps the
+// chip busy by itself and more of them crowd each other (one, two and four
+// chains: closed room, 7.4 M paths 18.3, 18.8 and 21.6 ms; eight Cornell
+// views, 1.5 M paths, 5.9, 6.6 and 6.6 ms; terrain 1080p, 64 frames 84.8, 84.9
+// and 85.8 ms, one frame 5.70, 5.59 and 5.62 ms -- but 6.5 ms when the two
+// streams share a hardware queue, which a process with several contexts sees).
+constexpr uint32_t kMaxChains = 1;
 constexpr uint32_t kChainPaths = 1000000u;
-constexpr uint32_t kChainLcm = 12;
+constexpr uint32_t kChainLcm = 1;
 
 // Chains of a launch of `paths` paths (one when `one` is set).
 inline uint32_t chain_count(uint64_t paths, bool one) {

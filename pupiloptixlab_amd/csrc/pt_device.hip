@@ -125,7 +125,7 @@ __device__ __forceinline__ bool trace_one(const DeviceBvh &bvh, uint2 *lds_col, 
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
-// Queue counters of one chain: for each bounce b the size of its extension
+// Queue counters of a launch: for each bounce b the size of its extension
 // queue and that of the shadow queue its traversal launch takes along (the
 // shadow rays of bounce b - 1), side by side so that shading reserves in both
 // with one atomic; then the cursors of the traversal launches.
@@ -142,8 +142,8 @@ constexpr uint32_t counter_count(uint32_t max_depth) { return 4u * (max_depth + 
 // queue: wave counts meet in LDS, one 64-bit atomic per block reserves slots
 // in both, and each lane gets its rank.  Every shading wave of a launch
 // counts into the same word, which the memory side serves one after another,
-// 4-5 ns each: with an atomic per wave and queue they bound the kernel.  Alone
-// (one chain), 16 bounces: a closed room at 8.3 M paths 19.2 -> 8.7 ms, now
+// 4-5 ns each: with an atomic per wave and queue they bound the kernel.  At
+// 16 bounces: a closed room at 8.3 M paths 19.2 -> 8.7 ms, now
 // bound by its queue traffic (4.2 TB/s), and the terrain at 33 M paths 11.9 ->
 // 5.2 ms, now by VALU issue.  All threads of the block must call it.
 struct QueueSlots {
@@ -200,14 +200,11 @@ __device__ __forceinline__ uint32_t tiled_pixel(uint32_t j, uint32_t w, uint32_t
     return h8 * w + (j - rw * h8);
 }
 
-// One chain of a launch: frames [frame0, frame0 + frames) of the pixels at
-// places [pix0, pix0 + pixels) of the tile order; frame f of the launch
-// draws from random-stream key frame_seed0 + f.
+// Frame f of the launch draws from random-stream key frame_seed0 + f.
 __global__ void k_raygen(PathQueue q, CameraRec cam, uint32_t width, uint32_t height, uint32_t frames,
-                         uint32_t frame_seed0, uint32_t *counters, uint32_t num_counters, uint32_t frame0,
-                         uint32_t pix0, uint32_t pixels) {
+                         uint32_t frame_seed0, uint32_t *counters, uint32_t num_counters) {
     const uint32_t npix = width * height;
-    const uint32_t total = pixels * frames;
+    const uint32_t total = npix * frames;
     const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
     if (tid == 0) {
         counters[0] = total;
@@ -215,7 +212,7 @@ __global__ void k_raygen(PathQueue q, CameraRec cam, uint32_t width, uint32_t he
     }
     for (uint32_t i = tid; i < total; i += gridDim.x * blockDim.x) {
         uint32_t f, place;
-        chain_slot(frame0, frames, pix0, i, f, place);
+        chain_slot(0u, frames, 0u, i, f, place);
         const uint32_t pixel = tiled_pixel(place, width, height);
         const uint32_t x = pixel % width, y = pixel / width;
         Rng rng = rng_init(pixel, frame_seed0 + f);
@@ -499,7 +496,7 @@ __device__ __forceinline__ bool guide_query_of(const GuideView &G, const PathQue
 //   k_guide_bin_scan first place of each cell, in blocks of kBinBlock cells
 //   k_guide_bin_move positions and slots to their places
 // Outputs go to the queries' own slots, so what is computed does not change.
-// Closed room 960x540, 16 frames, one chain: 69.5 M queries 27.8 -> 17.2 ms
+// Closed room 960x540, 16 frames: 69.5 M queries 27.8 -> 17.2 ms
 // (5.1 ms of it k_guide_bin, at 14 G atomics/s; the network itself 10.3 ms at
 // 56% VALU use instead of 23%).
 constexpr uint32_t kBinBits = 18, kBinBlock = 1024, kBinBlocks = (1u << kBinBits) / kBinBlock;
@@ -511,7 +508,7 @@ struct GuideBins {
     float4 *rec;       // per place: normalized position, slot
     uint32_t axis_bits;
 };
-// Words of one chain's cells; a launch's total sits after the blocks.
+// Words of the cells; a launch's total sits after the blocks.
 constexpr size_t kBinWords = (2u << kBinBits) + kBinBlocks + 64u;
 // Queues of at least this many slots are sorted; at 58 K the three small
 // launches per bounce just pay for themselves (a training frame 4.75 -> 4.70
@@ -815,13 +812,9 @@ __global__ void k_accumulate(const float4 *out_l, float4 *accum, float4 *frame, 
 
 // --- batched views ----------------------------------------------------------------
 // main.cu:39-78 for every (view, frame, pixel) of a batched launch.
-// Chain `chain` of `chains` takes the launch's slots [lo, hi) with
-// lo = total * chain / chains, into its own queue part.
 __global__ void k_raygen_batch(PathQueue q, const LaunchDesc *ld, const BatchViewDev *views, uint32_t path_bits,
-                               uint32_t *counters, uint32_t num_counters, uint32_t chain, uint32_t chains) {
-    const uint32_t all = ld->total_paths;
-    const uint32_t lo = batch_chain_begin(all, chain, chains);
-    const uint32_t total = batch_chain_begin(all, chain + 1, chains) - lo;
+                               uint32_t *counters, uint32_t num_counters) {
+    const uint32_t total = ld->total_paths;
     const uint32_t ns = ld->n_segs;
     const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
     if (tid == 0) {
@@ -829,17 +822,16 @@ __global__ void k_raygen_batch(PathQueue q, const LaunchDesc *ld, const BatchVie
         for (uint32_t i = 1; i < num_counters; ++i) counters[i] = 0u;
     }
     for (uint32_t i = tid; i < total; i += gridDim.x * blockDim.x) {
-        // The segment holding launch slot g; within a segment (consecutive
+        // The segment holding launch slot i; within a segment (consecutive
         // frames of one view) frames are interleaved as in k_raygen.
-        const uint32_t g = lo + i;
         uint32_t a = 0, z = ns - 1;
         while (a < z) {
             const uint32_t mid = (a + z + 1u) >> 1;
-            if (ld->e[ld->g[mid].first_entry].path_begin <= g) a = mid;
+            if (ld->e[ld->g[mid].first_entry].path_begin <= i) a = mid;
             else z = mid - 1u;
         }
         const LaunchSeg &sg = ld->g[a];
-        const uint32_t local = g - ld->e[sg.first_entry].path_begin;
+        const uint32_t local = i - ld->e[sg.first_entry].path_begin;
         const LaunchEntry en = ld->e[sg.first_entry + local % sg.frames];
         const uint32_t view = en.view & kEntryViewMask;
         const BatchViewDev &v = views[view];
@@ -1255,11 +1247,6 @@ struct ShapeHost {
 struct pt_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
-    // Streams of the second to fourth chains of a launch (pt_render and
-    // batched launches); dep_events fork them from and join them to the pass
-    // stream.
-    hipStream_t stream2 = nullptr, stream3 = nullptr, stream4 = nullptr;
-    std::vector<hipEvent_t> dep_events;
     std::string error;
     int num_cu = 256;
     uint32_t trace_blocks_per_cu = 8;       // resident traversal blocks per CU, sphere variant
@@ -1357,8 +1344,8 @@ struct pt_ctx {
     GuideState guide;
     uint4 *d_gout = nullptr;  // network outputs per queue slot
     uint32_t gout_cap = 0;
-    // Spatial order of the queries: cells of each chain, per queue slot cell
-    // and rank, sorted records.
+    // Spatial order of the queries: cells, per queue slot cell and rank,
+    // sorted records.
     uint32_t *d_bins = nullptr;
     uint2 *d_bin_where = nullptr;
     float4 *d_bin_rec = nullptr;
@@ -1550,8 +1537,7 @@ int ensure_queues(pt_ctx *ctx, uint32_t paths, uint32_t max_depth) {
     PT_HIP(hipMalloc((void **)&ctx->sq.s1, n * sizeof(float4)));
     PT_HIP(hipMalloc((void **)&ctx->sq.s2, n * sizeof(float4)));
     PT_HIP(hipMalloc((void **)&ctx->d_out_l, n * sizeof(float4)));
-    // One set of counters per chain of a pt_render launch (four at most).
-    PT_HIP(hipMalloc((void **)&ctx->d_counters, 4 * need_counters * sizeof(uint32_t)));
+    PT_HIP(hipMalloc((void **)&ctx->d_counters, need_counters * sizeof(uint32_t)));
     ctx->capacity = paths;
     ctx->num_counters = need_counters;
     return PT_OK;
@@ -1560,7 +1546,7 @@ int ensure_queues(pt_ctx *ctx, uint32_t paths, uint32_t max_depth) {
 uint32_t trace_grid(pt_ctx *ctx) {
     return (uint32_t)ctx->num_cu * (ctx->num_spheres > 0 ? ctx->trace_blocks_per_cu : ctx->trace_blocks_per_cu_tri);
 }
-// Shading grid for a chain of `paths` queue slots: a block for every 256 of
+// Shading grid for a launch of `paths` queue slots: a block for every 256 of
 // them, at most kShadeRounds times the blocks that can be resident at once.
 // Every block strides over the queue; with many more blocks than slots the
 // dispatcher balances uneven shading work across CUs, and blocks that find no
@@ -1581,33 +1567,12 @@ int ensure_spill(pt_ctx *ctx) {
         (uint32_t)ctx->num_cu * std::max(ctx->trace_blocks_per_cu, ctx->trace_blocks_per_cu_tri) * kTraceBlock;
     if (ctx->d_spill && ctx->spill_threads >= threads) return PT_OK;
     dfree(ctx->d_spill);
-    // Four areas: one per chain of a launch.
-    PT_HIP(hipMalloc((void **)&ctx->d_spill, 4 * (size_t)threads * kSpillEntries * sizeof(uint2)));
+    PT_HIP(hipMalloc((void **)&ctx->d_spill, (size_t)threads * kSpillEntries * sizeof(uint2)));
     ctx->spill_threads = threads;
     return PT_OK;
 }
 
 DeviceBvh device_bvh(pt_ctx *ctx) { return DeviceBvh{ctx->d_nodes, ctx->d_leaf, ctx->d_spill}; }
-// The tree with the spill area of chain `area` of a launch.
-DeviceBvh device_bvh_area(pt_ctx *ctx, uint32_t area) {
-    return DeviceBvh{ctx->d_nodes, ctx->d_leaf, ctx->d_spill + (size_t)area * ctx->spill_threads * kSpillEntries};
-}
-PathQueue queue_at(const PathQueue &q, size_t off) {
-    return PathQueue{q.ray0 + off, q.ray1 + off, q.tl + off, q.lr + off, q.hit + off};
-}
-ShadowQueue shadow_queue_at(const ShadowQueue &q, size_t off) { return ShadowQueue{q.s0 + off, q.s1 + off, q.s2 + off}; }
-
-// Events ordering the streams of a render: the fork and the joins of a
-// launch's chains.
-int ensure_dep_events(pt_ctx *ctx, uint32_t n) {
-    while (ctx->dep_events.size() < n) {
-        hipEvent_t e = nullptr;
-        PT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        ctx->dep_events.push_back(e);
-    }
-    return PT_OK;
-}
-
 // Network outputs and sorting buffers for `paths` queue slots.
 int ensure_guide_outputs(pt_ctx *ctx, uint32_t paths) {
     if (ctx->gout_cap >= paths) return PT_OK;
@@ -1619,29 +1584,28 @@ int ensure_guide_outputs(pt_ctx *ctx, uint32_t paths) {
     PT_HIP(hipMalloc((void **)&ctx->d_bin_where, (size_t)paths * sizeof(uint2)));
     PT_HIP(hipMalloc((void **)&ctx->d_bin_rec, (size_t)paths * sizeof(float4)));
     if (!ctx->d_bins) {
-        const size_t words = (size_t)kMaxChains * kBinWords;
-        PT_HIP(hipMalloc((void **)&ctx->d_bins, words * sizeof(uint32_t)));
-        PT_HIP(hipMemset(ctx->d_bins, 0, words * sizeof(uint32_t)));
+        PT_HIP(hipMalloc((void **)&ctx->d_bins, kBinWords * sizeof(uint32_t)));
+        PT_HIP(hipMemset(ctx->d_bins, 0, kBinWords * sizeof(uint32_t)));
     }
     ctx->gout_cap = paths;
     return PT_OK;
 }
 
-// Sorting buffers of chain `chain`, whose queue part starts at slot `slot0`.
-GuideBins guide_bins(const pt_ctx *ctx, uint32_t chain, size_t slot0, uint32_t grids) {
-    uint32_t *w = ctx->d_bins + (size_t)chain * kBinWords;
-    uint32_t grid_bits = 0;
+GuideBins guide_bins(const pt_ctx *ctx, uint32_t grids) {
+    uint32_t *w = ctx->d_bins, grid_bits = 0;
     while ((1u << grid_bits) < grids) ++grid_bits;
-    return GuideBins{w, w + (1u << kBinBits), w + (2u << kBinBits), ctx->d_bin_where + slot0, ctx->d_bin_rec + slot0,
+    return GuideBins{w, w + (1u << kBinBits), w + (2u << kBinBits), ctx->d_bin_where, ctx->d_bin_rec,
                      (kBinBits - grid_bits) / 3u};
 }
 
-// Network inference for a chain's extension queue of at most `paths` slots.
-void launch_guide_infer(const pt_ctx *ctx, hipStream_t stream, const GuideView &gv, const PathQueue &q,
-                        const uint32_t *count, uint4 *gout, uint32_t path_bits, const InferScene &sc,
-                        const GuideBins &bins, uint32_t paths) {
+// Network inference for an extension queue of at most `paths` slots.
+void launch_guide_infer(const pt_ctx *ctx, const GuideView &gv, const PathQueue &q, const uint32_t *count,
+                        uint32_t path_bits, const SceneView &sv, uint32_t paths) {
+    const hipStream_t stream = ctx->stream;
+    const InferScene sc{sv.tri, sv.shapes, sv.spheres, sv.materials};
+    const GuideBins bins = guide_bins(ctx, gv.grids);
     const dim3 grid(std::max(8u, ((uint32_t)ctx->num_cu * ctx->infer_blocks_per_cu) & ~7u)), block(kInferBlock);
-    uint2 *out = reinterpret_cast<uint2 *>(gout);
+    uint2 *out = reinterpret_cast<uint2 *>(ctx->d_gout);
     if (paths < kBinMinPaths) {
         hipLaunchKernelGGL(k_guide_infer<false>, grid, block, 0, stream, gv, q, count, out, ctx->d_stat + 4, path_bits,
                            sc, bins);
@@ -1686,10 +1650,9 @@ hipEvent_t next_event(pt_ctx *ctx) {
 // read after the render's final synchronization, so timing adds no host
 // synchronization inside the timed region.
 // A kernel kind's time is the union of its timers' intervals (the time
-// during which at least one of its dispatches ran; kernels of concurrent
-// chains overlap), and its launch count the number of distinct groups: timers
-// sharing a nonzero `group` (the same bounce of the chains of one pt_render
-// launch) count as one launch.
+// during which at least one of its dispatches ran), and its launch count the
+// number of distinct groups: timers sharing a nonzero `group` count as one
+// launch.
 constexpr uint64_t kGroupSingle = 1ull << 63;  // groups of single timers
 struct EventTimer {
     pt_ctx *ctx;
@@ -2341,6 +2304,7 @@ int bvh_refit(pt_ctx *ctx) {
 struct BatchShape {
     uint32_t capacity, shade_block, shade_bpc, trace_bpc;
     uint32_t train_paths;  // training launch width (0 = kTrainLaunchPaths)
+    uint32_t widest = 0;   // paths of the render's widest launch (0: capacity)
 };
 
 // Training samples for `steps` optimizer steps of `batch` samples (capped at
@@ -2366,15 +2330,7 @@ struct BatchGuide {
     uint32_t step = 0;    // optimizer steps taken on the ring
 };
 
-// The kernels of one launch (the sequence a hipGraph captures).  As in
-// pt_render, the launch's paths run as concurrent chains, each on its own
-// stream with its own queue part (a fixed share of the queues: slot ranges
-// come from the device launch descriptor), counters and spill area; under
-// capture the chains fork from and join the pass stream through events, so
-// the graph holds them as parallel branches.  Accumulation follows the join.
-// Needs ensure_dep_events(ctx, kMaxChains) and queues of batch_queue_paths.
-uint32_t batch_chains(const BatchShape &sh) { return chain_count(sh.capacity, false); }
-uint32_t batch_queue_paths(const BatchShape &sh) { return batch_queue_slots(sh.capacity); }
+// The kernels of one launch (the sequence a hipGraph captures).
 void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth, const ShadeParams &sp,
                           uint32_t path_bits, bool fp64, const BatchGuide &bg, bool timing = false,
                           uint64_t launch_group = 0) {
@@ -2396,91 +2352,53 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
     AovBuffers aov{nullptr, nullptr, nullptr, nullptr, 0u, 1u};
     const uint32_t tg = (uint32_t)ctx->num_cu * sh.trace_bpc;
     const uint32_t sg = (uint32_t)ctx->num_cu * sh.shade_bpc;
-    const uint32_t nchain = batch_chains(sh);
-    const size_t share = batch_share(batch_queue_paths(sh), nchain);  // queue slots per chain
-    const hipStream_t streams[] = {ctx->stream, ctx->stream2, ctx->stream3, ctx->stream4};
-    struct Chain {
-        hipStream_t stream;
-        uint32_t *counters;
-        PathQueue q[2];
-        ShadowQueue sq;
-        DeviceBvh bvh;
-        GuideShadeArgs ga;
-        uint4 *gout;
-        GuideBins bins;
-    } ch[kMaxChains];
-    for (uint32_t c = 0; c < nchain; ++c) {
-        Chain &k = ch[c];
-        k.stream = streams[c];
-        k.counters = ctx->d_counters + (size_t)c * ctx->num_counters;
-        k.q[0] = queue_at(ctx->q[0], c * share);
-        k.q[1] = queue_at(ctx->q[1], c * share);
-        k.sq = shadow_queue_at(ctx->sq, c * share);
-        k.bvh = DeviceBvh{b.d_nodes, b.d_leaf, ctx->d_spill + (size_t)c * ctx->spill_threads * kSpillEntries};
-        k.gout = ctx->d_gout ? ctx->d_gout + 6 * c * share : nullptr;
-        if (bg.infer) k.bins = guide_bins(ctx, c, c * share, (uint32_t)b.views.size());
-        k.ga = bg.ga;
-    }
-    if (nchain > 1) (void)hipEventRecord(ctx->dep_events[0], ctx->stream);
-    for (uint32_t c = 1; c < nchain; ++c) (void)hipStreamWaitEvent(ch[c].stream, ctx->dep_events[0], 0);
-    for (uint32_t c = 0; c < nchain; ++c)
-        hipLaunchKernelGGL(k_raygen_batch, dim3((uint32_t)ctx->num_cu * 32u), dim3(256), 0, ch[c].stream, ch[c].q[0],
-                           b.d_launch, b.d_views, path_bits, ch[c].counters, ctx->num_counters, c, nchain);
+    uint32_t *counters = ctx->d_counters;
+    const DeviceBvh bvh{b.d_nodes, b.d_leaf, ctx->d_spill};
+    hipLaunchKernelGGL(k_raygen_batch, dim3((uint32_t)ctx->num_cu * 32u), dim3(256), 0, ctx->stream, ctx->q[0],
+                       b.d_launch, b.d_views, path_bits, counters, ctx->num_counters);
     // The traversal of bounce bb's extension rays, with the shadow rays of the
     // bounce before it.
     const TraceKernel tk = trace_kernel(false, !b.spheres.empty());
-    auto trace = [&](const Chain &k, uint32_t bb, bool shadow) {
-        EventTimer t(ctx, timing, k.stream, launch_group ? (launch_group | (bb + 1)) : 0u);
-        uint32_t *pair = k.counters + counter_pair(bb);
-        const TraceJob job{k.q[bb & 1], pair, k.sq, shadow ? pair + 1 : nullptr, ctx->d_out_l,
-                           k.counters + counter_cursor(max_depth, bb), ctx->d_stat, b.d_roots, path_bits};
-        hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, k.stream, job, k.bvh);
+    auto trace = [&](uint32_t bb) {
+        EventTimer t(ctx, timing, nullptr, launch_group ? (launch_group | (bb + 1)) : 0u);
+        uint32_t *pair = counters + counter_pair(bb);
+        const TraceJob job{ctx->q[bb & 1], pair, ctx->sq, bb ? pair + 1 : nullptr, ctx->d_out_l,
+                           counters + counter_cursor(max_depth, bb), ctx->d_stat, b.d_roots, path_bits};
+        hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, ctx->stream, job, bvh);
         t.stop(kKindTrace);
     };
-    for (uint32_t c = 0; c < nchain; ++c) trace(ch[c], 0, false);
-    int cur = 0;
+    trace(0);
     for (uint32_t bb = 0; bb < max_depth; ++bb) {
-        const int nxt = cur ^ 1;
+        const PathQueue &in = ctx->q[bb & 1], &out = ctx->q[(bb & 1) ^ 1];
+        const uint32_t *count = counters + counter_pair(bb);
+        uint32_t *counts_out = counters + counter_pair(bb + 1);
         const uint64_t group = launch_group ? (launch_group | (bb + 1)) : 0u;
-        const bool infer_here = bg.infer && bb < bg.gdepth && bb + 1 < max_depth;
-        for (uint32_t c = 0; c < nchain; ++c) {
-            const Chain &k = ch[c];
-            if (bg.infer || bg.train) {
-                GuideShadeArgs ga = k.ga;
-                ga.gout = infer_here ? k.gout : nullptr;
-                if (infer_here) {
-                    EventTimer t(ctx, timing, k.stream, group);
-                    launch_guide_infer(ctx, k.stream, bg.view, k.q[cur], k.counters + counter_pair(bb), k.gout,
-                                       path_bits, InferScene{sv.tri, sv.shapes, sv.spheres, sv.materials}, k.bins,
-                                       (uint32_t)share);
-                    t.stop(kKindGuideInfer);
-                }
-                EventTimer t(ctx, timing, k.stream, group);
-                hipLaunchKernelGGL(k_shade_guided<true>, dim3((uint32_t)ctx->num_cu * sh.shade_bpc), dim3(256), 0,
-                                   k.stream, sv, sp, k.q[cur], k.counters + counter_pair(bb), k.q[nxt],
-                                   k.counters + counter_pair(bb + 1), k.sq, ctx->d_out_l, aov, ga, (const BatchViewDev *)b.d_views, path_bits,
-                                   (const LaunchDesc *)b.d_launch);
-                t.stop(kKindShade);
-            } else {
-                EventTimer t(ctx, timing, k.stream, group);
-                hipLaunchKernelGGL(shade_kernel(true, b.feat), dim3(sg), dim3(sh.shade_block), 0, k.stream, sv, sp,
-                                   k.q[cur], k.counters + counter_pair(bb), k.q[nxt],
-                                   k.counters + counter_pair(bb + 1), k.sq, ctx->d_out_l, aov,
-                                   (const BatchViewDev *)b.d_views, path_bits);
-                t.stop(kKindShade);
+        if (bg.infer || bg.train) {
+            const bool infer_here = bg.infer && bb < bg.gdepth && bb + 1 < max_depth;
+            GuideShadeArgs ga = bg.ga;
+            ga.gout = infer_here ? ctx->d_gout : nullptr;
+            if (infer_here) {
+                EventTimer t(ctx, timing, nullptr, group);
+                launch_guide_infer(ctx, bg.view, in, count, path_bits, sv, sh.widest ? sh.widest : sh.capacity);
+                t.stop(kKindGuideInfer);
             }
-            if (bb + 1 < max_depth) trace(k, bb + 1, true);
+            EventTimer t(ctx, timing, nullptr, group);
+            hipLaunchKernelGGL(k_shade_guided<true>, dim3(sg), dim3(256), 0, ctx->stream, sv, sp, in, count, out,
+                               counts_out, ctx->sq, ctx->d_out_l, aov, ga, (const BatchViewDev *)b.d_views, path_bits,
+                               (const LaunchDesc *)b.d_launch);
+            t.stop(kKindShade);
+        } else {
+            EventTimer t(ctx, timing, nullptr, group);
+            hipLaunchKernelGGL(shade_kernel(true, b.feat), dim3(sg), dim3(sh.shade_block), 0, ctx->stream, sv, sp, in,
+                               count, out, counts_out, ctx->sq, ctx->d_out_l, aov, (const BatchViewDev *)b.d_views,
+                               path_bits);
+            t.stop(kKindShade);
         }
-        cur = nxt;
-    }
-    for (uint32_t c = 1; c < nchain; ++c) {
-        (void)hipEventRecord(ctx->dep_events[c], ch[c].stream);
-        (void)hipStreamWaitEvent(ctx->stream, ctx->dep_events[c], 0);
+        if (bb + 1 < max_depth) trace(bb + 1);
     }
     hipLaunchKernelGGL(k_accumulate_batch, dim3((uint32_t)ctx->num_cu * 16u), dim3(256), 0, ctx->stream,
                        ctx->d_out_l, b.d_launch, b.d_views, fp64 ? 1u : 0u);
-    for (uint32_t c = 0; c < nchain; ++c)
-        hipLaunchKernelGGL(k_batch_count, dim3(1), dim3(64), 0, ctx->stream, ch[c].counters, max_depth, b.d_rays);
+    hipLaunchKernelGGL(k_batch_count, dim3(1), dim3(64), 0, ctx->stream, counters, max_depth, b.d_rays);
 }
 
 // Width of a launch of guide-training frames: by default at most 2^23 paths
@@ -2519,7 +2437,7 @@ int batch_guide_setup(pt_ctx *ctx, const pt_batch_params &p, const BatchShape &s
     bg.ga.fixed_c = std::min(gs.cfg.fixed_selection, 1.f);
     bg.gdepth = gs.cfg.guided_depth ? gs.cfg.guided_depth : max_depth;
     if (bg.infer) {
-        const int rc = ensure_guide_outputs(ctx, batch_queue_paths(sh));
+        const int rc = ensure_guide_outputs(ctx, sh.capacity);
         if (rc != PT_OK) return rc;
         bg.ga.gout = ctx->d_gout;
     }
@@ -2566,8 +2484,7 @@ int batch_guide_setup(pt_ctx *ctx, const pt_batch_params &p, const BatchShape &s
 
 // Renders the batch's frames with one launch shape.  Returns PT_OK and the
 // wall time in *ms.
-int batch_run(pt_ctx *ctx, const pt_batch_params &p, const BatchShape &sh, bool graph, double *ms,
-              uint32_t *launches) {
+int batch_run(pt_ctx *ctx, const pt_batch_params &p, BatchShape sh, bool graph, double *ms, uint32_t *launches) {
     BatchState &b = ctx->batch;
     const auto t0 = std::chrono::steady_clock::now();
     int rc = batch_upload(ctx);
@@ -2583,7 +2500,7 @@ int batch_run(pt_ctx *ctx, const pt_batch_params &p, const BatchShape &sh, bool 
                      "path-id range";
         return PT_ERR_CAPACITY;
     }
-    if ((rc = ensure_queues(ctx, batch_queue_paths(sh), max_depth)) != PT_OK) return rc;
+    if ((rc = ensure_queues(ctx, sh.capacity, max_depth)) != PT_OK) return rc;
     if ((rc = ensure_spill(ctx)) != PT_OK) return rc;
     BatchGuide bg;
     bg.infer = (p.render_flags & PT_RENDER_GUIDE) != 0;
@@ -2599,6 +2516,8 @@ int batch_run(pt_ctx *ctx, const pt_batch_params &p, const BatchShape &sh, bool 
     const uint32_t train_cap = batch_train_capacity(b, sh);
     std::vector<LaunchDesc> plan;
     batch_plan(b.views, sh.capacity, true, plan, ps, train_cap, gate);
+    if (!gate)  // (which may plan wider launches later)
+        for (const LaunchDesc &l : plan) sh.widest = std::max(sh.widest, l.total_paths);
     if (bg.train && b.gate_views < b.views.size()) {
         dfree(b.d_gate_acc);
         dfree(b.d_gate_off);
@@ -2628,7 +2547,6 @@ int batch_run(pt_ctx *ctx, const pt_batch_params &p, const BatchShape &sh, bool 
     spar.aov = 0;
     const bool fp64 = (p.render_flags & PT_RENDER_FP64_ACCUM) != 0;
     if ((rc = batch_guide_setup(ctx, p, sh, max_depth, plan, bg)) != PT_OK) return rc;
-    if ((rc = ensure_dep_events(ctx, kMaxChains)) != PT_OK) return rc;
     // Per-kernel event timing (direct launches only; around the training
     // steps in both modes).
     const bool timing = (p.render_flags & PT_RENDER_TIMING) != 0;
@@ -2852,15 +2770,6 @@ int pt_create(int hip_device, pt_ctx **out) {
         delete ctx;
         return PT_ERR_HIP;
     }
-    if (hipStreamCreateWithFlags(&ctx->stream2, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&ctx->stream3, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&ctx->stream4, hipStreamNonBlocking) != hipSuccess) {
-        g_create_error = "failed to create the chain streams";
-        for (hipStream_t st : {ctx->stream, ctx->stream2, ctx->stream3})
-            if (st) (void)hipStreamDestroy(st);
-        delete ctx;
-        return PT_ERR_HIP;
-    }
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, hip_device) == hipSuccess && prop.multiProcessorCount > 0)
         ctx->num_cu = prop.multiProcessorCount;
@@ -2909,8 +2818,6 @@ void pt_destroy(pt_ctx *ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    for (hipStream_t st : {ctx->stream2, ctx->stream3, ctx->stream4})
-        if (st) (void)hipStreamSynchronize(st);
     ctx->guide.release();
     batch_free_all(ctx);
     free_scene(ctx);
@@ -2924,9 +2831,7 @@ void pt_destroy(pt_ctx *ctx) {
     dfree(ctx->d_refit_err);
     dfree(ctx->d_count_hist);
     for (hipEvent_t e : ctx->event_pool) (void)hipEventDestroy(e);
-    for (hipEvent_t e : ctx->dep_events) (void)hipEventDestroy(e);
-    for (hipStream_t st : {ctx->stream4, ctx->stream3, ctx->stream2, ctx->stream})
-        if (st) (void)hipStreamDestroy(st);
+    if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
 
@@ -3418,7 +3323,6 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
 
     const bool timing = (p->flags & PT_RENDER_TIMING) != 0;
     const SceneView sv = scene_view(ctx);
-    if ((rc = ensure_dep_events(ctx, 4)) != PT_OK) return rc;  // fork and the joins of the chains
     ShadeParams sp;
     sp.max_depth = max_depth;
     sp.rr_depth = p->rr_depth;
@@ -3427,7 +3331,7 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
     const uint32_t tg = trace_grid(ctx);
 
     const uint32_t batches = (p->spp + per_launch - 1) / per_launch;
-    const uint32_t hist_elems = std::max(1u, batches) * 4u * ctx->num_counters;  // one set per chain
+    const uint32_t hist_elems = std::max(1u, batches) * ctx->num_counters;
     if (hist_elems > ctx->count_hist_slots || !ctx->d_count_hist) {
         dfree(ctx->d_count_hist);
         PT_HIP(hipMalloc((void **)&ctx->d_count_hist, (size_t)hist_elems * sizeof(uint32_t)));
@@ -3460,32 +3364,12 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
             return PT_ERR_HIP;
     }
 
-    // Chains: a launch's queue slots are split into up to kMaxChains
-    // contiguous ranges of at least kChainPaths (10^6) paths, each traced, shaded and
-    // shadow-tested on its own stream with its own part of the queues, its
-    // own counters and spill area.  A chain's bounces serialize and every
-    // kernel drains before the next starts; the other chains fill the idle
-    // CUs meanwhile.  Terrain 1080p, one chain against four: 815 -> 970
-    // Msamples/s at 20 frames per launch, 861 -> 1058-1071 at 64.  More
-    // streams than the hardware queues (four) cost: two chains with a second
-    // stream each for their shadow rays reached 885 and 967, three such 743.
-    // Every path's work is unchanged, so is the image.
     uint32_t done = 0, batch = 0;
     uint32_t sample_cnt = ctx->sample_cnt, seed = ctx->random_seed;
-    std::vector<uint32_t> chains_per_launch;
     const uint32_t gdepth = ctx->guide.cfg.guided_depth ? ctx->guide.cfg.guided_depth : max_depth;
-    const hipStream_t chain_stream[] = {ctx->stream, ctx->stream2, ctx->stream3, ctx->stream4};
     while (done < p->spp) {
         const uint32_t frames = std::min(per_launch, p->spp - done);
         const uint32_t total = frames * npix;
-        const uint32_t nchain = chain_count(total, (p->flags & PT_RENDER_ONE_CHAIN) != 0);
-        // With at least as many frames as chains, a chain takes a share of the
-        // frames of every pixel, so the chains run through the same pixels at
-        // the same time and share L2 (terrain 1080p, four chains of 5 frames:
-        // 968 Msamples/s at 20 frames per launch, against 914 for four bands
-        // of pixels in all 20 frames); otherwise a band of pixels.
-        ChainPart part[kMaxChains];
-        chain_parts(frames, npix, nchain, part);
         AovBuffers aov{nullptr, nullptr, nullptr, nullptr, frames - 1, npix};
         if (sp.aov) {
             aov.albedo = ctx->d_albedo;
@@ -3503,109 +3387,68 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
             ga.rs.max_depth = max_depth;
             ga.rs.epoch = gs.epoch;
         }
-        struct Chain {
-            uint32_t frame0, frames, pix0, pixels;  // frames x tile-order pixel places of the launch
-            uint32_t slot0, paths;                  // its slots [slot0, slot0 + paths) of the queues
-            uint32_t shade_grid;
-            hipStream_t stream;
-            uint32_t *counters;
-            PathQueue q[2];
-            ShadowQueue sq;
-            DeviceBvh bvh;
-            uint4 *gout;
-            GuideBins bins;
-        } ch[kMaxChains];
-        for (uint32_t c = 0; c < nchain; ++c) {
-            Chain &k = ch[c];
-            k.frame0 = part[c].frame0;
-            k.frames = part[c].frames;
-            k.pix0 = part[c].pix0;
-            k.pixels = part[c].pixels;
-            k.slot0 = part[c].slot0;
-            k.paths = part[c].paths;
-            k.shade_grid = shade_grid(ctx, guided, guide_train, k.paths);
-            k.stream = chain_stream[c];
-            k.counters = ctx->d_counters + (size_t)c * ctx->num_counters;
-            k.q[0] = queue_at(ctx->q[0], k.slot0);
-            k.q[1] = queue_at(ctx->q[1], k.slot0);
-            k.sq = shadow_queue_at(ctx->sq, k.slot0);
-            k.bvh = device_bvh_area(ctx, c);
-            k.gout = ctx->d_gout ? ctx->d_gout + 6 * (size_t)k.slot0 : nullptr;
-            if (guide_infer) k.bins = guide_bins(ctx, c, k.slot0, 1u);
-        }
-        // The other chains start after everything before on the pass stream.
-        if (nchain > 1) PT_HIP(hipEventRecord(ctx->dep_events[0], ctx->stream));
-        for (uint32_t c = 1; c < nchain; ++c) PT_HIP(hipStreamWaitEvent(ch[c].stream, ctx->dep_events[0], 0));
-        // Timer groups: a bounce's kernels of all chains time as one launch.
+        uint32_t *counters = ctx->d_counters;
+        const DeviceBvh bvh = device_bvh(ctx);
+        const uint32_t sg = shade_grid(ctx, guided, guide_train, total);
+        // Timer groups: a bounce's kernels of one kind time as one launch.
         const uint64_t launch_group = (uint64_t)(batch + 1) << 16;
-        for (uint32_t c = 0; c < nchain; ++c) {
-            const Chain &k = ch[c];
-            EventTimer t(ctx, timing, k.stream, launch_group | 0xFFFFu);
-            const uint32_t grid = std::min<uint32_t>((k.paths + 255) / 256, (uint32_t)ctx->num_cu * 32u);
-            hipLaunchKernelGGL(k_raygen, dim3(grid), dim3(256), 0, k.stream, k.q[0], ctx->camera, ctx->width,
-                               ctx->height, k.frames, seed, k.counters, ctx->num_counters, k.frame0, k.pix0, k.pixels);
+        {
+            EventTimer t(ctx, timing, nullptr, launch_group | 0xFFFFu);
+            const uint32_t grid = std::min<uint32_t>((total + 255) / 256, (uint32_t)ctx->num_cu * 32u);
+            hipLaunchKernelGGL(k_raygen, dim3(grid), dim3(256), 0, ctx->stream, ctx->q[0], ctx->camera, ctx->width,
+                               ctx->height, frames, seed, counters, ctx->num_counters);
             t.stop(kKindRaygen);
         }
         // The traversal of bounce b's extension rays together with the shadow
         // rays of the bounce before it (the last bounce casts none), or in
         // launches of their own when kernels are to be timed alone.
         const TraceKernel tk = trace_kernel(ctx->counting, ctx->num_spheres > 0);
-        auto trace = [&](const Chain &k, uint32_t b, bool shadow) {
-            uint32_t *pair = k.counters + counter_pair(b);
-            TraceJob job{k.q[b & 1], pair, k.sq, shadow ? pair + 1 : nullptr, ctx->d_out_l,
-                         k.counters + counter_cursor(max_depth, b), ctx->d_stat, nullptr, 31u};
-            if (shadow && (p->flags & PT_RENDER_ONE_CHAIN)) {
+        auto trace = [&](uint32_t b) {
+            uint32_t *pair = counters + counter_pair(b);
+            TraceJob job{ctx->q[b & 1], pair, ctx->sq, b ? pair + 1 : nullptr, ctx->d_out_l,
+                         counters + counter_cursor(max_depth, b), ctx->d_stat, nullptr, 31u};
+            if (b && (p->flags & PT_RENDER_ONE_CHAIN)) {
                 TraceJob sj = job;
                 sj.ext_count = nullptr;
-                sj.work = k.counters + counter_shadow_cursor(max_depth, b);
-                EventTimer t(ctx, timing, k.stream, launch_group | b);
-                hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, k.stream, sj, k.bvh);
+                sj.work = counters + counter_shadow_cursor(max_depth, b);
+                EventTimer t(ctx, timing, nullptr, launch_group | b);
+                hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, ctx->stream, sj, bvh);
                 t.stop(kKindShadow);
                 job.shd_count = nullptr;
             }
-            EventTimer t(ctx, timing, k.stream, launch_group | (b + 1));
-            hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, k.stream, job, k.bvh);
+            EventTimer t(ctx, timing, nullptr, launch_group | (b + 1));
+            hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, ctx->stream, job, bvh);
             t.stop(kKindTrace);
         };
-        for (uint32_t c = 0; c < nchain; ++c) trace(ch[c], 0, false);
-        int cur = 0;
+        trace(0);
         for (uint32_t b = 0; b < max_depth; ++b) {
-            const int nxt = cur ^ 1;
+            const PathQueue &in = ctx->q[b & 1], &out = ctx->q[(b & 1) ^ 1];
+            const uint32_t *count = counters + counter_pair(b);
+            uint32_t *counts_out = counters + counter_pair(b + 1);
             // The guide is sampled at vertices b < guided_depth; the vertex of
             // the last bounce never samples a direction.
             const bool infer_here = guide_infer && b < gdepth && b + 1 < max_depth;
             const uint64_t group = launch_group | (b + 1);
-            for (uint32_t c = 0; c < nchain; ++c) {
-                const Chain &k = ch[c];
-                GuideShadeArgs gac = ga;
-                gac.gout = infer_here ? k.gout : nullptr;
-                if (infer_here) {
-                    EventTimer t(ctx, timing, k.stream, group);
-                    launch_guide_infer(ctx, k.stream, gview, k.q[cur], k.counters + counter_pair(b), k.gout, 31u,
-                                       InferScene{sv.tri, sv.shapes, sv.spheres, sv.materials}, k.bins, k.paths);
-                    t.stop(kKindGuideInfer);
-                }
-                {
-                    EventTimer t(ctx, timing, k.stream, group);
-                    if (guided)
-                        hipLaunchKernelGGL(k_shade_guided<false>, dim3(k.shade_grid), dim3(256), 0, k.stream, sv, sp, k.q[cur],
-                                           k.counters + counter_pair(b), k.q[nxt], k.counters + counter_pair(b + 1),
-                                           k.sq, ctx->d_out_l, aov, gac,
-                                           (const BatchViewDev *)nullptr, 31u, (const LaunchDesc *)nullptr);
-                    else
-                        hipLaunchKernelGGL(shade_kernel(false, ctx->shade_feat), dim3(k.shade_grid), dim3(256), 0, k.stream, sv,
-                                           sp, k.q[cur], k.counters + counter_pair(b), k.q[nxt],
-                                           k.counters + counter_pair(b + 1), k.sq, ctx->d_out_l, aov,
-                                           (const BatchViewDev *)nullptr, 31u);
-                    t.stop(kKindShade);
-                }
-                if (b + 1 < max_depth) trace(k, b + 1, true);
+            GuideShadeArgs gac = ga;
+            gac.gout = infer_here ? ctx->d_gout : nullptr;
+            if (infer_here) {
+                EventTimer t(ctx, timing, nullptr, group);
+                launch_guide_infer(ctx, gview, in, count, 31u, sv, total);
+                t.stop(kKindGuideInfer);
             }
-            cur = nxt;
-        }
-        for (uint32_t c = 1; c < nchain; ++c) {
-            PT_HIP(hipEventRecord(ctx->dep_events[c], ch[c].stream));
-            PT_HIP(hipStreamWaitEvent(ctx->stream, ctx->dep_events[c], 0));
+            {
+                EventTimer t(ctx, timing, nullptr, group);
+                if (guided)
+                    hipLaunchKernelGGL(k_shade_guided<false>, dim3(sg), dim3(256), 0, ctx->stream, sv, sp, in, count, out,
+                                       counts_out, ctx->sq, ctx->d_out_l, aov, gac, (const BatchViewDev *)nullptr, 31u,
+                                       (const LaunchDesc *)nullptr);
+                else
+                    hipLaunchKernelGGL(shade_kernel(false, ctx->shade_feat), dim3(sg), dim3(256), 0, ctx->stream, sv,
+                                       sp, in, count, out, counts_out, ctx->sq, ctx->d_out_l, aov,
+                                       (const BatchViewDev *)nullptr, 31u);
+                t.stop(kKindShade);
+            }
+            if (b + 1 < max_depth) trace(b + 1);
         }
         {
             EventTimer t(ctx, timing);
@@ -3631,29 +3474,26 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
             t.stop(kKindGuide);
         }
         PT_HIP(hipGetLastError());
-        // Keep this launch's queue counters (both chains' sets); read back once
-        // after the last launch.
-        PT_HIP(hipMemcpyAsync(ctx->d_count_hist + (size_t)batch * kMaxChains * ctx->num_counters, ctx->d_counters,
-                              (size_t)nchain * ctx->num_counters * sizeof(uint32_t), hipMemcpyDeviceToDevice,
-                              ctx->stream));
-        chains_per_launch.push_back(nchain);
+        // Keep this launch's queue counters; read back once after the last
+        // launch.
+        PT_HIP(hipMemcpyAsync(ctx->d_count_hist + (size_t)batch * ctx->num_counters, counters,
+                              (size_t)ctx->num_counters * sizeof(uint32_t), hipMemcpyDeviceToDevice, ctx->stream));
         if (p->accumulate) sample_cnt += frames;
         seed += frames;
         done += frames;
         ++batch;
     }
-    std::vector<uint32_t> hist((size_t)batch * kMaxChains * ctx->num_counters);
+    std::vector<uint32_t> hist((size_t)batch * ctx->num_counters);
     PT_HIP(hipMemcpyAsync(hist.data(), ctx->d_count_hist, hist.size() * sizeof(uint32_t), hipMemcpyDeviceToHost,
                           ctx->stream));
     PT_HIP(hipStreamSynchronize(ctx->stream));
-    for (uint32_t k = 0; k < batch; ++k)
-        for (uint32_t c = 0; c < chains_per_launch[k]; ++c) {
-            const uint32_t *cn = hist.data() + ((size_t)k * kMaxChains + c) * ctx->num_counters;
-            for (uint32_t b = 0; b < max_depth; ++b) {
-                ctx->stats.rays_extension += cn[counter_pair(b)];
-                ctx->stats.rays_shadow += cn[counter_pair(b + 1) + 1];
-            }
+    for (uint32_t k = 0; k < batch; ++k) {
+        const uint32_t *cn = hist.data() + (size_t)k * ctx->num_counters;
+        for (uint32_t b = 0; b < max_depth; ++b) {
+            ctx->stats.rays_extension += cn[counter_pair(b)];
+            ctx->stats.rays_shadow += cn[counter_pair(b + 1) + 1];
         }
+    }
     if (guide_infer) {
         unsigned long long nq = 0;
         PT_HIP(hipMemcpy(&nq, ctx->d_stat + 4, sizeof(nq), hipMemcpyDeviceToHost));
@@ -3793,7 +3633,7 @@ int pt_render_noalloc(pt_ctx *ctx, const pt_render_params *p) {
         // k_raygen clears every counter before the first traversal reads them.
         const uint32_t rgrid = std::min<uint32_t>((total + 255) / 256, (uint32_t)ctx->num_cu * 32u);
         hipLaunchKernelGGL(k_raygen, dim3(rgrid), dim3(256), 0, ctx->stream, L.q[0], ctx->camera, ctx->width,
-                           ctx->height, frames, seed, L.counters, num_counters, 0u, 0u, npix);
+                           ctx->height, frames, seed, L.counters, num_counters);
         AovBuffers aov{nullptr, nullptr, nullptr, nullptr, frames - 1, npix};
         if (sp.aov) {
             aov.albedo = ctx->d_albedo;
@@ -4387,7 +4227,7 @@ static int pt_batch_autotune_unguarded(pt_ctx *ctx, const pt_batch_params *param
         ns = ms * 1e6 / (double)probe_paths;
         return PT_OK;
     };
-    BatchShape best{kBatchDefaultPaths, 256u, 8u, ctx->trace_blocks_per_cu, params->train_paths_per_launch};
+    BatchShape best{kBatchDefaultPaths, 256u, 8u, ctx->trace_blocks_per_cu, params->train_paths_per_launch, 0u};
     best.capacity = std::min(best.capacity, 1u << path_bits);
     best.capacity = std::max(best.capacity, max_npix);
     double best_ns = 0.0, dummy = 0.0, default_ns = 0.0;
