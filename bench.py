@@ -515,8 +515,6 @@ def measured_traffic(frames_per_launch):
         t = json.load(f)
     scale = frames_per_launch / t["frames_per_launch"]
     note = None if scale == 1 else f"scaled from {t['frames_per_launch']}-frame launches x {scale:.3f}"
-    if t.get("chains", 1) > 1:  # an earlier version's launches, with shadow rays traced apart
-        note = f"{note + ', ' if note else ''}taken with {t['chains']} chains per launch, extension rays alone"
     return {k: v.get("hbm_bytes_per_launch", v["hbm_bytes_per_dispatch"]) * scale
             for k, v in t["kernels"].items()}, note
 
