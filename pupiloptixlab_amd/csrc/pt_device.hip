@@ -1584,8 +1584,15 @@ int ensure_guide_outputs(pt_ctx *ctx, uint32_t paths) {
     PT_HIP(hipMalloc((void **)&ctx->d_bin_where, (size_t)paths * sizeof(uint2)));
     PT_HIP(hipMalloc((void **)&ctx->d_bin_rec, (size_t)paths * sizeof(float4)));
     if (!ctx->d_bins) {
-        PT_HIP(hipMalloc((void **)&ctx->d_bins, kBinWords * sizeof(uint32_t)));
-        PT_HIP(hipMemset(ctx->d_bins, 0, kBinWords * sizeof(uint32_t)));
+        // Every sort takes a histogram of zeros and leaves one.  The first is
+        // cleared in the order of the stream that sorts, which does not wait
+        // for the null stream; without a clear there are no bins.
+        uint32_t *bins = nullptr;
+        PT_HIP(hipMalloc((void **)&bins, kBinWords * sizeof(uint32_t)));
+        const hipError_t e = hipMemsetAsync(bins, 0, kBinWords * sizeof(uint32_t), ctx->stream);
+        if (e != hipSuccess) (void)hipFree(bins);
+        PT_HIP(e);
+        ctx->d_bins = bins;
     }
     ctx->gout_cap = paths;
     return PT_OK;

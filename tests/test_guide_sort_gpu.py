@@ -57,3 +57,22 @@ def test_batch_grids(tracer, views):
         assert np.array_equal(a, b)
     tracer.guide_disable()
     tracer.batch_clear()
+
+
+def test_first_sort_of_a_context():
+    """The histogram's first clear is ordered before the first sort, whatever
+    the memory held: contexts made where others left their queues, sorted
+    inference first thing."""
+    scene = pt.HostScene.generate(pt.SCENE_DOOR_ROOM, seed=3, width=257, height=160)
+    want = None
+    for k, per in enumerate((1, 2, 2, 2)):
+        print(f"case: context {k}, {per} frames per launch at once", flush=True)
+        with pt.PathTracer(0) as t:
+            t.set_scene(scene)
+            t.build_bvh()
+            t.guide_enable(log2_table=14)
+            t.guide_set_params(*params(1))
+            t.render(spp=2, mis_mode=pt.MIS_CONSISTENT, guide=True, spp_per_launch=per)
+            got = t.read(pt.BUF_ACCUM)
+        want = got if want is None else want
+        assert np.array_equal(got, want)
