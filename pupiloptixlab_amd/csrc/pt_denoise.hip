@@ -31,6 +31,7 @@
 // the call with its read-back 3390 -> 2570 us.
 #include <hip/hip_runtime.h>
 
+#include <cfloat>
 #include <cmath>
 
 #include "pt_denoise.h"
@@ -61,6 +62,11 @@ __device__ __forceinline__ f3 demodulate(f3 c, f3 a) {
     return mk3(c.x / fmaxf(a.x, kDenoiseAlbedoEps), c.y / fmaxf(a.y, kDenoiseAlbedoEps),
                c.z / fmaxf(a.z, kDenoiseAlbedoEps));
 }
+
+// 1 / sigma^2 of the albedo weight.  Finite, so that equal albedos weigh 1: the
+// reciprocal overflows for sigma below 5.4e-20, where only differences under
+// 1e-18 weigh anything else than 0.
+__device__ __forceinline__ float inverse_square(float sigma) { return fminf(1.f / (sigma * sigma), FLT_MAX); }
 
 // e^-x as one exp2 (argument and result each rounded once).
 __device__ __forceinline__ float exp_neg(float x) { return __builtin_amdgcn_exp2f(x * -1.44269504088896341f); }
@@ -176,7 +182,7 @@ __global__ __launch_bounds__(256) void k_dn_prepare(const float4 *in, Guides g, 
     int x0, y0;
     if (!wave_place<kRows>(w, h, 0u, blocks, x0, y0)) return;
     const int x = min(x0 + (int)__lane_id(), (int)w - 1);
-    const float inv_albedo = 1.f / (prm.sigma_albedo * prm.sigma_albedo);
+    const float inv_albedo = inverse_square(prm.sigma_albedo);
     GuideValue gp[kRows];
     // Moments about the center's luminance: their difference loses nothing
     // where the window is flat.
@@ -235,7 +241,7 @@ __global__ __launch_bounds__(256) void k_dn_atrous(const float4 *in, Guides g, f
     if (!wave_place<kRows>(w, h, log2_step, blocks, x0, y0)) return;
     const int step = 1 << log2_step, lane = (int)__lane_id();
     const int x = min(x0 + lane, (int)w - 1);
-    const float inv_albedo = 1.f / (prm.sigma_albedo * prm.sigma_albedo);
+    const float inv_albedo = inverse_square(prm.sigma_albedo);
     GuideValue gp[kRows];
     float l0[kRows], inv_sigma[kRows], sv[kRows], sw[kRows];
     f3 sc[kRows];

@@ -50,3 +50,18 @@ def test_pixels_that_are_not_finite_reach_their_windows_only(tracer, w, h):
     near = np.zeros((h, w), bool)  # 2 pixels of taps see the variance of 1 more, taken from windows of 2 more
     near[4:15, 15:26] = near[25:36, 65:76] = True
     assert np.array_equal(got[~near], clean[~near])
+
+
+# Sigmas whose square is below the float range (or zero in it): pixels of the
+# same albedo blend, others do not, as in 64 bits.  No weight but the
+# luminance's is rounded here, so the bound above holds.
+@pytest.mark.gpu
+@pytest.mark.parametrize("sigma", [1e-19, 1e-20, 3e-22, 1e-30])
+@pytest.mark.parametrize("w,h", [(63, 33), (1000, 502)])
+def test_albedo_scales_down_to_nothing(tracer, w, h, sigma):
+    print(f"case: denoise {w}x{h} sigma_albedo={sigma}", flush=True)
+    rgba, a, n = images(w, h, 7)
+    a = np.where(a > 0.225, np.float32(0.25), np.float32(0.2))
+    got = tracer.denoise_image(rgba, a, n, sigma_albedo=sigma)
+    want = dn.denoise(rgba, a, n, sigma_albedo=sigma)
+    assert np.allclose(got, want, rtol=2e-4, atol=1e-5)
