@@ -124,6 +124,7 @@ __device__ __forceinline__ GuideValue load_guides(const Guides &g, size_t p) {
     if constexpr (kNormal != kNoNormal) {
         v.n = load3(g.normal, p);
         v.bare = dot(v.n, v.n) == 0.f;
+        if (v.bare) v.n = mk3(0.f);  // also where only the square is zero: no weight against a surface
     }
     if constexpr (kAlbedo) v.a = load3(g.albedo, p);
     return v;

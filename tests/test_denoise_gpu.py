@@ -65,3 +65,16 @@ def test_albedo_scales_down_to_nothing(tracer, w, h, sigma):
     got = tracer.denoise_image(rgba, a, n, sigma_albedo=sigma)
     want = dn.denoise(rgba, a, n, sigma_albedo=sigma)
     assert np.allclose(got, want, rtol=2e-4, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exponent", [64.0, 1.0, 0.01])
+@pytest.mark.parametrize("w,h", [(63, 33), (1000, 502)])
+def test_normals_without_length_are_no_surface(tracer, w, h, exponent):
+    """A normal whose squared length underflows marks a pixel without a surface as a zero one does, bit for bit."""
+    print(f"case: denoise {w}x{h} normals of 1e-24, exponent {exponent}", flush=True)
+    rgba, a, n = images(w, h, 8)
+    bare = ~n.any(-1)
+    tiny = np.where(bare[..., None], np.float32(1e-24), n)
+    assert np.array_equal(tracer.denoise_image(rgba, a, tiny, sigma_normal=exponent),
+                          tracer.denoise_image(rgba, a, n, sigma_normal=exponent))
