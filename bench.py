@@ -501,7 +501,7 @@ def summarize_pmc(fetch_dir, write_dir, frames_per_launch, out_path, kernels, ch
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_terrain_1080p.json")
-TRAFFIC_KERNELS = {"trace": "k_trace<false, false>", "shade": "k_shade<false, "}
+TRAFFIC_KERNELS = {"trace": "k_trace<false", "shade": "k_shade<false, "}
 
 
 def measured_traffic(frames_per_launch):

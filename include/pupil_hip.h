@@ -299,7 +299,9 @@ int pt_render_noalloc(pt_ctx *ctx, const pt_render_params *params);
 /* BufferManager::GetBuffer + device-to-host copy (system/buffer.cpp:34-99). */
 int pt_read_buffer(pt_ctx *ctx, int which, void *host_dst, size_t bytes);
 int pt_get_stats(pt_ctx *ctx, pt_stats *out);
-/* Node-visit / triangle-test counting in the traversal kernels (off by default). */
+/* Node-visit / triangle-test counting (off by default): renders then walk each
+ * ray by itself, so that the counts are the rays' own, the same on every run and
+ * for any launch width.  The image is the same; rendering is slower. */
 int pt_set_counting(pt_ctx *ctx, int enable);
 /* Last error text of the context (or of the last failed pt_create when ctx is NULL). */
 const char *pt_last_error(const pt_ctx *ctx);

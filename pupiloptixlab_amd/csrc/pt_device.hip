@@ -267,6 +267,20 @@ __device__ __forceinline__ void add_contribution(const TraceJob &j, uint32_t i) 
     }
 }
 
+__device__ __forceinline__ void fetch_ray(const TraceJob &j, uint32_t ne, uint32_t i, f3 &o, f3 &d, float &tmax,
+                                          uint32_t &root, bool &any_hit) {
+    any_hit = i >= ne;
+    const float4 a = any_hit ? j.sq.s0[i - ne] : j.q.ray0[i], b = any_hit ? j.sq.s1[i - ne] : j.q.ray1[i];
+    o = f3of(a);
+    d = f3of(b);
+    tmax = any_hit ? a.w : kMaxDistance;
+    root = j.roots ? j.roots[(any_hit ? f2u(b.w) & 0x7FFFFFFFu : f2u(a.w)) >> j.path_bits] : 0u;
+}
+__device__ __forceinline__ void finish_ray(const TraceJob &j, uint32_t ne, uint32_t i, bool any_hit, const Hit &h) {
+    if (!any_hit) j.q.hit[i] = make_float4(h.t, u2f(h.prim), h.b1, h.b2);
+    else if (h.prim == kMissPrim) add_contribution(j, i - ne);
+}
+
 // Persistent grid sized to the resident occupancy (trace_stream).  A bounce's
 // shadow rays go into the launch of the next bounce's extension rays (their
 // results are read only by the shading after it): the tail of one kind of
@@ -277,12 +291,11 @@ __device__ __forceinline__ void add_contribution(const TraceJob &j, uint32_t i) 
 // 6.89 ms, 2.4 M triangles 1080p 64 frames 117.1 -> 114.7 ms).
 // Six waves per SIMD for triangles, five with the sphere test: registers and
 // the 12.5 KB of LDS per block allow as many.
-template <bool kCount, bool kSph>
+template <bool kSph>
 __global__ __launch_bounds__(kTraceBlock, kSph ? 5 : 6) void k_trace(TraceJob j, DeviceBvh bvh) {
     __shared__ StreamLds<kLdsStack> lds[kTraceBlock / 64];
     const uint32_t ne = j.ext_count ? *j.ext_count : 0u, ns = j.shd_count ? *j.shd_count : 0u;
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
-    TraverseStats ste{0, 0}, sts{0, 0};
     const uint32_t total = ne + ns, waves = gridDim.x * (kTraceBlock / 64);
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid >> 6));
     // Chunks of a quarter of a wave's even share, 64 to 256 rays: the cursor is
@@ -292,25 +305,38 @@ __global__ __launch_bounds__(kTraceBlock, kSph ? 5 : 6) void k_trace(TraceJob j,
     LdsStack stack(reinterpret_cast<uint2 *>(&L.stack[0][lane_id()]), bvh.spill + (size_t)gtid * kSpillEntries, 64u);
     auto load_node = [&](uint32_t i, NodeWords &n) { load_node_words(bvh.nodes, i, n); };
     auto fetch = [&](uint32_t i, f3 &o, f3 &d, float &tmax, uint32_t &root, bool &any_hit) {
-        any_hit = i >= ne;
-        const float4 a = any_hit ? j.sq.s0[i - ne] : j.q.ray0[i], b = any_hit ? j.sq.s1[i - ne] : j.q.ray1[i];
-        o = f3of(a);
-        d = f3of(b);
-        tmax = any_hit ? a.w : kMaxDistance;
-        root = j.roots ? j.roots[(any_hit ? f2u(b.w) & 0x7FFFFFFFu : f2u(a.w)) >> j.path_bits] : 0u;
+        fetch_ray(j, ne, i, o, d, tmax, root, any_hit);
     };
-    auto finish = [&](uint32_t i, bool any_hit, const Hit &h) {
-        if (!any_hit) j.q.hit[i] = make_float4(h.t, u2f(h.prim), h.b1, h.b2);
-        else if (h.prim == kMissPrim) add_contribution(j, i - ne);
-    };
-    trace_stream<kCount, kSph>(L, stack, bvh.tris, load_node, total, chunk, wave, waves, j.work, kExtTmin,
-                               kShadowEps, fetch, finish, ste, sts);
-    if (kCount) {
-        atomicAdd(j.stat + 0, (unsigned long long)ste.nodes);
-        atomicAdd(j.stat + 1, (unsigned long long)ste.tris);
-        atomicAdd(j.stat + 2, (unsigned long long)sts.nodes);
-        atomicAdd(j.stat + 3, (unsigned long long)sts.tris);
+    auto finish = [&](uint32_t i, bool any_hit, const Hit &h) { finish_ray(j, ne, i, any_hit, h); };
+    trace_stream<kSph>(L, stack, bvh.tris, load_node, total, chunk, wave, waves, j.work, kExtTmin, kShadowEps, fetch,
+                       finish);
+}
+
+// The counting form of k_trace: each ray walks by itself and tests leaves
+// where it finds them, so that the visits and tests counted are the ray's own.
+// In k_trace they depend on which rays share a wave, as rays walk on past hits
+// among their waiting pairs.  The hits are the same.
+template <bool kSph>
+__global__ __launch_bounds__(kTraceBlock) void k_trace_counted(TraceJob j, DeviceBvh bvh) {
+    __shared__ uint2 lds[kLdsStack * kTraceBlock];
+    const uint32_t ne = j.ext_count ? *j.ext_count : 0u, ns = j.shd_count ? *j.shd_count : 0u;
+    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
+    TraverseStats ste{0, 0}, sts{0, 0};
+    for (uint32_t i = gtid; i < ne + ns; i += gridDim.x * blockDim.x) {
+        f3 o, d;
+        float tmax;
+        uint32_t root;
+        bool any_hit;
+        fetch_ray(j, ne, i, o, d, tmax, root, any_hit);
+        Hit h;
+        if (any_hit) trace_one<true, true, kSph>(bvh, lds + threadIdx.x, gtid, o, d, kShadowEps, tmax, h, sts, root);
+        else trace_one<false, true, kSph>(bvh, lds + threadIdx.x, gtid, o, d, kExtTmin, tmax, h, ste, root);
+        finish_ray(j, ne, i, any_hit, h);
     }
+    atomicAdd(j.stat + 0, (unsigned long long)ste.nodes);
+    atomicAdd(j.stat + 1, (unsigned long long)ste.tris);
+    atomicAdd(j.stat + 2, (unsigned long long)sts.nodes);
+    atomicAdd(j.stat + 3, (unsigned long long)sts.tris);
 }
 
 // --- shading -----------------------------------------------------------------------
@@ -1052,14 +1078,13 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_rays(const float *rays, u
     }
 }
 
-// Traversal variants: counting on/off x sphere leaves present/absent (a
+// Traversal kernels: counting or not x sphere leaves present/absent (a
 // triangle-only tree runs without the sphere test, like an OptiX pipeline
 // built without the sphere primitive flag, optix/pipeline.cpp:14-28).
 using TraceKernel = void (*)(TraceJob, DeviceBvh);
 using TraceRaysKernel = void (*)(const float *, uint32_t, DeviceBvh, uint4 *);
 TraceKernel trace_kernel(bool count, bool sph) {
-    return count ? (sph ? k_trace<true, true> : k_trace<true, false>)
-                 : (sph ? k_trace<false, true> : k_trace<false, false>);
+    return count ? (sph ? k_trace_counted<true> : k_trace_counted<false>) : (sph ? k_trace<true> : k_trace<false>);
 }
 using ShadeKernel = void (*)(SceneView, ShadeParams, PathQueue, const uint32_t *, PathQueue, uint32_t *, ShadowQueue,
                             float4 *, AovBuffers, const BatchViewDev *, uint32_t);
@@ -2788,8 +2813,8 @@ int pt_create(int hip_device, pt_ctx **out) {
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kTraceBlock, 0) == hipSuccess && n > 0)
                 out = (uint32_t)n;
         };
-        resident(reinterpret_cast<const void *>(k_trace<false, true>), ctx->trace_blocks_per_cu);
-        resident(reinterpret_cast<const void *>(k_trace<false, false>), ctx->trace_blocks_per_cu_tri);
+        resident(reinterpret_cast<const void *>(k_trace<true>), ctx->trace_blocks_per_cu);
+        resident(reinterpret_cast<const void *>(k_trace<false>), ctx->trace_blocks_per_cu_tri);
         int c = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, k_guide_infer<true>, kInferBlock, 0) == hipSuccess && c > 0)
             ctx->infer_blocks_per_cu = (uint32_t)c;

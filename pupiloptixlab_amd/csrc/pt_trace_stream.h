@@ -66,12 +66,11 @@ constexpr uint32_t kFlushPairs = 40;
 // closest-hit and at `any_tmin` for any-hit rays, both positive.
 // finish(i, any_hit, hit) takes its result (any-hit rays: only whether there
 // is a hit).
-template <bool kCount, bool kSph, int kEntries, typename Stack, typename LoadNode, typename Fetch, typename Finish>
+template <bool kSph, int kEntries, typename Stack, typename LoadNode, typename Fetch, typename Finish>
 __device__ __forceinline__ void trace_stream(StreamLds<kEntries> &L, Stack stack, const LeafTri *tris,
                                              LoadNode load_node, uint32_t total, uint32_t chunk,
                                              uint32_t wave, uint32_t waves, uint32_t *cursor, float ext_tmin,
-                                             float any_tmin, Fetch fetch, Finish finish, TraverseStats &ste,
-                                             TraverseStats &sts) {
+                                             float any_tmin, Fetch fetch, Finish finish) {
     const uint32_t lane = __lane_id();
     uint32_t next = wave * chunk, end = min(next + chunk, total);
     if (next >= total) return;
@@ -110,10 +109,6 @@ __device__ __forceinline__ void trace_stream(StreamLds<kEntries> &L, Stack stack
             const float4 *p = reinterpret_cast<const float4 *>(tris + pr.x);
             const float4 a = p[0], b = p[1], c = p[2];
             const float tmin = (cd & 64u) ? any_tmin : ext_tmin;
-            if (kCount) {
-                if (cd & 64u) sts.tris++;
-                else ste.tris++;
-            }
             float t;
             bool h;
             if (kSph && f2u(b.w) != 0u)
@@ -194,10 +189,6 @@ __device__ __forceinline__ void trace_stream(StreamLds<kEntries> &L, Stack stack
         // while pairs are tested.
         uint32_t t_base = 0, t_bits = 0;
         if (r.have) {
-            if (kCount) {
-                if (any_hit) sts.nodes++;
-                else ste.nodes++;
-            }
             trav_node(r, t_base, t_bits);
             uint32_t node_index = 0;
             r.have = trav_next(r, stack, node_index);

@@ -79,3 +79,29 @@ def test_more_rays_than_the_grid(tracer):
     tracer.reset()
     tracer.render(spp=5, spp_per_launch=1, one_chain=True)
     assert np.array_equal(a, tracer.read(pt.BUF_ACCUM))
+
+
+@pytest.mark.parametrize("spheres", [0, 24])
+def test_counts_are_the_rays_own(tracer, spheres):
+    """Node visits and primitive tests of the same frames do not depend on launch width, on which rays share a
+    launch or on the run, and counting does not change the image."""
+    print(f"case: counting, terrain 322x181 with {spheres} spheres, 4 frames", flush=True)
+    scene = pt.HostScene.generate(pt.SCENE_TERRAIN, seed=6, width=322, height=181, grid=128, spheres=spheres)
+    tracer.set_scene(scene)
+    tracer.build_bvh()
+    tracer.render(spp=4)
+    image = tracer.read(pt.BUF_ACCUM)
+    keys = ("rays_extension", "rays_shadow", "node_visits", "tri_tests", "shadow_node_visits", "shadow_tri_tests")
+    counts = []
+    tracer.set_counting(True)
+    try:
+        for per, one in ((4, False), (4, False), (4, True), (1, False), (3, True)):
+            tracer.reset()
+            before = tracer.stats()
+            tracer.render(spp=4, spp_per_launch=per, one_chain=one)
+            after = tracer.stats()
+            counts.append({k: after[k] - before[k] for k in keys})
+            assert np.array_equal(image, tracer.read(pt.BUF_ACCUM))
+    finally:
+        tracer.set_counting(False)
+    assert all(c == counts[0] for c in counts) and min(counts[0].values()) > 0
