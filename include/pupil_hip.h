@@ -221,9 +221,10 @@ typedef struct pt_stats {
     double ms_total;         /* wall time of pt_render calls */
     /* Per kernel kind, for launches made with PT_RENDER_TIMING: the time during
      * which at least one of its dispatches ran (HIP events) and the number of
-     * launches timed (one per bounce).  A bounce's shadow rays are traced in
-     * the launch of the next bounce's extension rays, which counts as trace;
-     * PT_RENDER_ONE_CHAIN traces them in launches of their own (ms_shadow). */
+     * launches timed (one per bounce; the last bounce casts no shadow rays).  A
+     * bounce's shadow rays are traced in the launch of the next bounce's
+     * extension rays, which counts for both kinds: their times overlap.
+     * PT_RENDER_ONE_CHAIN traces each kind in launches of its own. */
     double ms_raygen, ms_trace, ms_shade, ms_shadow, ms_accumulate;
     uint64_t launches_trace, launches_shade, launches_shadow;
     uint32_t bvh_nodes, bvh_leaf_tris, bvh_depth;

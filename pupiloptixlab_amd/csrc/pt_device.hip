@@ -1699,12 +1699,14 @@ struct EventTimer {
             if (a) (void)hipEventRecord(a, stream);
         }
     }
-    void stop(int kind) {
+    // `also`: a second kind whose work the launch takes along (or -1).
+    void stop(int kind, int also = -1) {
         if (!on || !a) return;
         hipEvent_t b = next_event(ctx);
         if (!b) return;
         (void)hipEventRecord(b, stream);
         ctx->pending.push_back(pt_ctx::Pending{kind, a, b, group});
+        if (also >= 0) ctx->pending.push_back(pt_ctx::Pending{also, a, b, group});
     }
 };
 
@@ -2397,7 +2399,7 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
         const TraceJob job{ctx->q[bb & 1], pair, ctx->sq, bb ? pair + 1 : nullptr, ctx->d_out_l,
                            counters + counter_cursor(max_depth, bb), ctx->d_stat, b.d_roots, path_bits};
         hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, ctx->stream, job, bvh);
-        t.stop(kKindTrace);
+        t.stop(kKindTrace, job.shd_count ? kKindShadow : -1);
     };
     trace(0);
     for (uint32_t bb = 0; bb < max_depth; ++bb) {
@@ -3450,7 +3452,7 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
             }
             EventTimer t(ctx, timing, nullptr, launch_group | (b + 1));
             hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, ctx->stream, job, bvh);
-            t.stop(kKindTrace);
+            t.stop(kKindTrace, job.shd_count ? kKindShadow : -1);
         };
         trace(0);
         for (uint32_t b = 0; b < max_depth; ++b) {

@@ -105,3 +105,31 @@ def test_counts_are_the_rays_own(tracer, spheres):
     finally:
         tracer.set_counting(False)
     assert all(c == counts[0] for c in counts) and min(counts[0].values()) > 0
+
+
+def test_times_of_launches_that_take_both_kinds_of_rays(tracer):
+    """Timed renders, direct batches too: a launch with extension and shadow rays counts for both kinds."""
+    print("case: timed renders of 2 launches at depth 6, shared and separate shadow launches, and a batch", flush=True)
+    scene = pt.HostScene.generate(pt.SCENE_CORNELL, width=160, height=120)
+    tracer.set_scene(scene)
+    tracer.build_bvh()
+    keys = ("ms_trace", "ms_shadow", "launches_trace", "launches_shadow")
+
+    def timed(call):
+        before = tracer.stats()
+        call()
+        after = tracer.stats()
+        return [after[k] - before[k] for k in keys]
+
+    for one in (False, True):
+        ms_trace, ms_shadow, n_trace, n_shadow = timed(
+            lambda: tracer.render(spp=4, max_depth=6, spp_per_launch=2, timing=True, one_chain=one))
+        assert (n_trace, n_shadow) == (2 * 6, 2 * 5)
+        assert 0.0 < ms_shadow and 0.0 < ms_trace
+        assert one or ms_shadow < ms_trace  # a part of the same launches
+    tracer.batch_clear()
+    tracer.batch_add_view(scene, 2)
+    ms_trace, ms_shadow, n_trace, n_shadow = timed(lambda: tracer.batch_render(graph=False, timing=True))
+    tracer.batch_clear()
+    depth = scene.desc.max_depth
+    assert n_trace % depth == 0 and n_shadow * depth == n_trace * (depth - 1) and 0.0 < ms_shadow < ms_trace
