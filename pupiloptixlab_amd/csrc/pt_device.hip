@@ -1374,6 +1374,7 @@ struct pt_ctx {
     uint32_t *d_bins = nullptr;
     uint2 *d_bin_where = nullptr;
     float4 *d_bin_rec = nullptr;
+    uint32_t bin_cap = 0;
     uint32_t infer_blocks_per_cu = 2;
 
     // batched views (pt_batch_*)
@@ -1598,29 +1599,45 @@ int ensure_spill(pt_ctx *ctx) {
 }
 
 DeviceBvh device_bvh(pt_ctx *ctx) { return DeviceBvh{ctx->d_nodes, ctx->d_leaf, ctx->d_spill}; }
-// Network outputs and sorting buffers for `paths` queue slots.
+// Network outputs for `paths` queue slots.
 int ensure_guide_outputs(pt_ctx *ctx, uint32_t paths) {
     if (ctx->gout_cap >= paths) return PT_OK;
     ctx->gout_cap = 0;
     dfree(ctx->d_gout);
+    PT_HIP(hipMalloc((void **)&ctx->d_gout, (size_t)paths * 6 * sizeof(uint4)));
+    ctx->gout_cap = paths;
+    return PT_OK;
+}
+
+// Sorting buffers for launches of up to `paths` paths (24 bytes per slot), for
+// those that are sorted.  Allocated after everything else a render needs: one
+// that memory does not suffice for takes its queries in queue order.
+void ensure_guide_bins(pt_ctx *ctx, uint32_t paths) {
+    if (paths < kBinMinPaths || ctx->bin_cap >= paths) return;
+    ctx->bin_cap = 0;
     dfree(ctx->d_bin_where);
     dfree(ctx->d_bin_rec);
-    PT_HIP(hipMalloc((void **)&ctx->d_gout, (size_t)paths * 6 * sizeof(uint4)));
-    PT_HIP(hipMalloc((void **)&ctx->d_bin_where, (size_t)paths * sizeof(uint2)));
-    PT_HIP(hipMalloc((void **)&ctx->d_bin_rec, (size_t)paths * sizeof(float4)));
-    if (!ctx->d_bins) {
+    bool ok = hipMalloc((void **)&ctx->d_bin_where, (size_t)paths * sizeof(uint2)) == hipSuccess &&
+              hipMalloc((void **)&ctx->d_bin_rec, (size_t)paths * sizeof(float4)) == hipSuccess;
+    if (ok && !ctx->d_bins) {
         // Every sort takes a histogram of zeros and leaves one.  The first is
         // cleared in the order of the stream that sorts, which does not wait
         // for the null stream; without a clear there are no bins.
         uint32_t *bins = nullptr;
-        PT_HIP(hipMalloc((void **)&bins, kBinWords * sizeof(uint32_t)));
-        const hipError_t e = hipMemsetAsync(bins, 0, kBinWords * sizeof(uint32_t), ctx->stream);
-        if (e != hipSuccess) (void)hipFree(bins);
-        PT_HIP(e);
-        ctx->d_bins = bins;
+        ok = hipMalloc((void **)&bins, kBinWords * sizeof(uint32_t)) == hipSuccess;
+        if (ok && hipMemsetAsync(bins, 0, kBinWords * sizeof(uint32_t), ctx->stream) != hipSuccess) {
+            (void)hipFree(bins);
+            ok = false;
+        }
+        if (ok) ctx->d_bins = bins;
     }
-    ctx->gout_cap = paths;
-    return PT_OK;
+    if (ok) {
+        ctx->bin_cap = paths;
+    } else {
+        dfree(ctx->d_bin_where);
+        dfree(ctx->d_bin_rec);
+        (void)hipGetLastError();  // not the render's error
+    }
 }
 
 GuideBins guide_bins(const pt_ctx *ctx, uint32_t grids) {
@@ -1638,7 +1655,7 @@ void launch_guide_infer(const pt_ctx *ctx, const GuideView &gv, const PathQueue 
     const GuideBins bins = guide_bins(ctx, gv.grids);
     const dim3 grid(std::max(8u, ((uint32_t)ctx->num_cu * ctx->infer_blocks_per_cu) & ~7u)), block(kInferBlock);
     uint2 *out = reinterpret_cast<uint2 *>(ctx->d_gout);
-    if (paths < kBinMinPaths) {
+    if (paths < kBinMinPaths || paths > ctx->bin_cap) {
         hipLaunchKernelGGL(k_guide_infer<false>, grid, block, 0, stream, gv, q, count, out, ctx->d_stat + 4, path_bits,
                            sc, bins);
         return;
@@ -2513,6 +2530,7 @@ int batch_guide_setup(pt_ctx *ctx, const pt_batch_params &p, const BatchShape &s
         bg.ga.rs.max_depth = max_depth;
         bg.ga.rs.epoch = 0;
     }
+    if (bg.infer) ensure_guide_bins(ctx, sh.widest ? sh.widest : sh.capacity);
     return PT_OK;
 }
 
@@ -3397,6 +3415,7 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
                                        ctx->error))
             return PT_ERR_HIP;
     }
+    if (guide_infer) ensure_guide_bins(ctx, per_launch * npix);
 
     uint32_t done = 0, batch = 0;
     uint32_t sample_cnt = ctx->sample_cnt, seed = ctx->random_seed;

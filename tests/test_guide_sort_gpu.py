@@ -2,6 +2,8 @@
 queries in queue order (smaller queues): each query's outputs go to its own
 slot, so the same frames in wide and in narrow launches give the same image,
 bit for bit, with one hash grid and with one per batch view."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -76,3 +78,25 @@ def test_first_sort_of_a_context():
             got = t.read(pt.BUF_ACCUM)
         want = got if want is None else want
         assert np.array_equal(got, want)
+
+
+def free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert pt.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_no_sorting_buffers_for_what_is_not_sorted():
+    """A guided batch with queues for 2^22 paths whose launches are narrow holds 96 bytes per slot for the network's
+    outputs and no more."""
+    slots = 1 << 22
+    print("case: guided batch, launches of 12 K paths in queues of 4 M", flush=True)
+    with pt.PathTracer(0) as t:
+        t.batch_add_view(pt.HostScene.generate(pt.SCENE_CORNELL_VARIANT, seed=1, triangles=2000, width=128, height=96), 1)
+        t.guide_enable_batch(log2_table=14)
+        t.guide_set_params(*params(2))
+        kw = {"mis_mode": pt.MIS_CONSISTENT, "paths_per_launch": slots, "graph": False}
+        t.batch_render(**kw)
+        before = free_bytes()
+        t.batch_render(guide=True, **kw)
+        assert before - free_bytes() < 96 * slots + (32 << 20)
