@@ -25,6 +25,7 @@ rays' kernel alone.  The CPU baseline is the oracle (scalar C++,
 multithreaded) on a bounded band of rows of the same frame.
 """
 import argparse
+import hashlib
 import json
 import os
 import sys
@@ -187,7 +188,7 @@ def batched_experiment(pt, views, seed):
 # Hash-table entries per level (log2) of the guided render judged at equal
 # time: a 4 MiB table (2^16 entries x 16 levels) makes inference faster, which
 # at equal time outweighs the larger table's accuracy on this workload (door
-# room 1080p, 256 training frames, four chains per launch: ratio 3.74-3.83 at
+# room 1080p, 256 training frames, when a launch ran as four chains: ratio 3.74-3.83 at
 # 2^16, 3.51-3.80 at 2^17, 3.64-3.66 at 2^18, 3.02-3.65 at 2^19, the
 # library's default).  The guided reference keeps the default.
 GUIDED_LOG2_TABLE = 16
@@ -456,13 +457,22 @@ def batched_guided_experiment(pt, n_door, n_terrain, width, height, door_ref_spp
     return out
 
 
+def kernel_sources():
+    """Digest of the sources of the kernels whose counters are summarized."""
+    h = hashlib.sha256()
+    for name in ("pt_device.hip", "pt_trace_stream.h", "pt_bvh.h", "pt_shade.h", "pt_bsdf.h", "pt_math.h"):
+        with open(os.path.join(ROOT, "pupiloptixlab_amd", "csrc", name), "rb") as f:
+            h.update(f.read())
+    return h.hexdigest()[:16]
+
+
 def summarize_pmc(fetch_dir, write_dir, frames_per_launch, out_path, kernels, chains=1):
     """Per-dispatch HBM bytes of each kernel from two rocprofv3 --pmc runs
     (FETCH_SIZE, WRITE_SIZE; KiB per dispatch), each scaled by the factor that
     maps the counter onto the known bytes of the copy-probe kernel.  The runs
-    render frames_per_launch frames per launch (the bench's launch shape) in
-    `chains` concurrent chains, so one bounce (a logical launch, the unit of
-    the bench's per-kernel figures) is `chains` dispatches of each kernel."""
+    render frames_per_launch frames per launch (the bench's launch shape); one
+    bounce (a logical launch, the unit of the bench's per-kernel figures) is
+    `chains` dispatches of each kernel, one unless a build splits launches."""
     import csv
     import glob
 
@@ -476,7 +486,8 @@ def summarize_pmc(fetch_dir, write_dir, frames_per_launch, out_path, kernels, ch
                     vals.setdefault(r["Kernel_Name"], []).append(float(r["Counter_Value"]))
         return vals
 
-    out = {"frames_per_launch": int(frames_per_launch), "chains": int(chains), "kernels": {}}
+    out = {"frames_per_launch": int(frames_per_launch), "chains": int(chains), "sources": kernel_sources(),
+           "kernels": {}}
     for counter, d, key in (("FETCH_SIZE", fetch_dir, "fetch"), ("WRITE_SIZE", write_dir, "write")):
         vals = per_kernel(d, counter)
         copy = [v for k, vs in vals.items() if "k_copy" in k for v in vs]
@@ -505,14 +516,17 @@ TRAFFIC_KERNELS = {"trace": "k_trace<false", "shade": "k_shade<false, "}
 
 
 def measured_traffic(frames_per_launch):
-    """HBM bytes per logical launch (one bounce, all chains) of each kernel
-    from the committed counter summary, for launches of frames_per_launch
-    frames: measured at that shape, or scaled linearly in frames from the
-    measured shape (marked so)."""
+    """HBM bytes per logical launch (one bounce) of each kernel from the
+    committed counter summary, for launches of frames_per_launch frames:
+    measured at that shape, or scaled linearly in frames from the measured
+    shape (marked so).  A summary of other sources counts for nothing: what it
+    measured is not what runs."""
     if not os.path.exists(TRAFFIC_FILE):
         return {}, None
     with open(TRAFFIC_FILE) as f:
         t = json.load(f)
+    if t.get("sources") != kernel_sources():
+        return {}, None
     scale = frames_per_launch / t["frames_per_launch"]
     note = None if scale == 1 else f"scaled from {t['frames_per_launch']}-frame launches x {scale:.3f}"
     return {k: v.get("hbm_bytes_per_launch", v["hbm_bytes_per_dispatch"]) * scale
@@ -684,7 +698,7 @@ def main():
     # What the counters say bounds the kernel: HBM bandwidth if its measured
     # traffic runs near the device's copy bandwidth, else latency and issue.
     if hbm_gbps is None:
-        limiter = "unmeasured (no counter summary)"
+        limiter = "unmeasured (no counter summary of these kernels)"
     elif hbm_gbps >= 0.6 * copy_gbps:
         limiter = f"hbm bandwidth (counter traffic {hbm_gbps:.0f} GB/s)"
     else:
@@ -744,7 +758,8 @@ def main():
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic,
-            "traffic_shape": traffic_note or f"measured at this launch shape ({frames_per_launch} frames per launch)",
+            "traffic_shape": None if traffic is None else
+                             traffic_note or f"measured at this launch shape ({frames_per_launch} frames per launch)",
             "traffic_GBps": hbm_gbps,
             "limiter": limiter,
             "single_chain": single_chain,

@@ -2,8 +2,8 @@
 reading back for the bench line's `traffic` field, on synthetic rocprofv3
 counter files (each counter is scaled by the factor that maps the copy
 probe's reading onto its known bytes, per-dispatch figures are averaged over
-a kernel's dispatches, and a bounce of a launch run as n concurrent chains is
-n dispatches); and the refusal of runs on more than one GPU."""
+a kernel's dispatches, a bounce of a launch run as n chains is n dispatches,
+and a summary of other kernel sources is not read); and the refusal of runs on more than one GPU."""
 import csv
 import json
 import os
@@ -60,6 +60,24 @@ def test_summary_scales_and_counts_chains(tmp_path, monkeypatch):
     assert note is None and same["trace"] == tr["hbm_bytes_per_launch"]
     half, note = bench.measured_traffic(10)
     assert note is not None and abs(half["trace"] - tr["hbm_bytes_per_launch"] / 2) < 1e-6
+
+
+def test_summary_of_other_sources_is_not_read(tmp_path, monkeypatch):
+    """Counters of kernels that have changed since are no counters of this build's."""
+    kib = bench.COPY_PROBE_BYTES / 1024.0
+    for name, counter in (("fetch", "FETCH_SIZE"), ("write", "WRITE_SIZE")):
+        write_counters(str(tmp_path / name), counter, [kib], {"trace": [1.0], "shade": [1.0], "shadow": [1.0]})
+    out = str(tmp_path / "traffic.json")
+    bench.summarize_pmc(str(tmp_path / "fetch"), str(tmp_path / "write"), 20, out, bench.TRAFFIC_KERNELS)
+    monkeypatch.setattr(bench, "TRAFFIC_FILE", out)
+    assert bench.measured_traffic(20)[0]["trace"] > 0
+    t = json.load(open(out))
+    for sources in ("0" * 16, None):
+        t["sources"] = sources
+        if sources is None:
+            del t["sources"]
+        json.dump(t, open(out, "w"))
+        assert bench.measured_traffic(20) == ({}, None)
 
 
 def test_bench_refuses_more_than_one_gpu():
