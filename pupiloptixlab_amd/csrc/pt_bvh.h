@@ -243,8 +243,9 @@ struct TraverseStats {
 //
 // The traversal of one ray is trav_init followed by trav_step until it
 // returns false; one step visits one node and tests its leaf primitives.
-// traverse_bvh runs a ray to the end; the GPU closest-hit kernel interleaves
-// rays per lane (a lane whose ray ends takes the next one).
+// traverse_bvh runs a ray to the end (host, ray queries, counting renders).
+// Renders on the GPU walk their rays by trav_node and trav_next and test the
+// primitives apart from the walk (pt_trace_stream.h).
 struct TravRay {
     f3 o, d;
     RayPre rp;

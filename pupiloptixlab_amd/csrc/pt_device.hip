@@ -25,7 +25,7 @@
 #include "../../include/pupil_hip.h"
 #include "pt_bvh.h"
 #include "pt_batch_plan.h"
-#include "pt_chains.h"
+#include "pt_slots.h"
 #include "pt_timing.h"
 #include "pt_trace_stream.h"
 #include "pt_bvh_build.h"
@@ -184,22 +184,9 @@ __device__ __forceinline__ f3 f3of(float4 v) { return mk3(v.x, v.y, v.z); }
 // camera rays nearly coincide, their later rays leave from nearly the same
 // points, and compaction keeps them together at later bounces (terrain
 // 1080p, against one frame after another: traversal 2.6% faster, launches
-// 1.7% faster at 20 frames and 2.1% at 64).  Tile order (tiled_pixel): full
-// 8x8 tiles first, then the pixels of a partial right strip and bottom strip
-// in row order.  The path id keeps frame and pixel (frame * pixels + pixel),
-// so films, AOVs and random streams do not depend on the order.
-__device__ __forceinline__ uint32_t tiled_pixel(uint32_t j, uint32_t w, uint32_t h) {
-    const uint32_t w8 = w & ~7u, h8 = h & ~7u, tiled = w8 * h8;
-    if (j < tiled) {
-        const uint32_t t = j >> 6, k = j & 63u, tiles_per_row = w8 >> 3;
-        return ((t / tiles_per_row) * 8u + (k >> 3)) * w + (t % tiles_per_row) * 8u + (k & 7u);
-    }
-    j -= tiled;
-    const uint32_t rw = w - w8;
-    if (j < rw * h8) return (j / rw) * w + w8 + j % rw;
-    return h8 * w + (j - rw * h8);
-}
-
+// 1.7% faster at 20 frames and 2.1% at 64).  The path id keeps frame and pixel
+// (frame * pixels + pixel), so films, AOVs and random streams do not depend on
+// the order.
 // Frame f of the launch draws from random-stream key frame_seed0 + f.
 __global__ void k_raygen(PathQueue q, CameraRec cam, uint32_t width, uint32_t height, uint32_t frames,
                          uint32_t frame_seed0, uint32_t *counters, uint32_t num_counters) {
@@ -212,7 +199,7 @@ __global__ void k_raygen(PathQueue q, CameraRec cam, uint32_t width, uint32_t he
     }
     for (uint32_t i = tid; i < total; i += gridDim.x * blockDim.x) {
         uint32_t f, place;
-        chain_slot(0u, frames, 0u, i, f, place);
+        frame_slot(frames, i, f, place);
         const uint32_t pixel = tiled_pixel(place, width, height);
         const uint32_t x = pixel % width, y = pixel / width;
         Rng rng = rng_init(pixel, frame_seed0 + f);
@@ -1062,7 +1049,10 @@ __global__ void k_copy(const float4 *__restrict__ src, float4 *__restrict__ dst,
         dst[i] = src[i];
 }
 
-// Closest-hit / any-hit over caller rays (pt_trace_rays).
+// Closest-hit / any-hit over caller rays (pt_trace_rays).  One ray per lane to
+// its end: each has its own tmin, zero and negative ones too, for which the
+// bits of t do not order as the floats do, as trace_stream's key needs.  0.32 of
+// the 3.2 ms that a call with 1 M rays takes.
 template <bool kAnyHit, bool kSph>
 __global__ __launch_bounds__(kTraceBlock) void k_trace_rays(const float *rays, uint32_t count, DeviceBvh bvh,
                                                             uint4 *hits) {
@@ -1271,6 +1261,12 @@ struct ShapeHost {
 
 struct pt_ctx {
     int device = 0;
+    // A launch's kernels follow one another here.  Its paths as two or four
+    // chains on streams of their own crowd each other: closed room at 7.4 M
+    // paths 18.3, 18.8 and 21.6 ms with one, two and four; eight Cornell views,
+    // 1.5 M paths, 5.9, 6.6 and 6.6 ms; terrain 1080p, 64 frames, 84.8, 84.9 and
+    // 85.8 ms, one frame 5.70, 5.59 and 5.62 ms, but 6.5 ms when two streams
+    // share a hardware queue, as in a process with several contexts.
     hipStream_t stream = nullptr;
     std::string error;
     int num_cu = 256;
@@ -1706,14 +1702,13 @@ constexpr uint64_t kGroupSingle = 1ull << 63;  // groups of single timers
 struct EventTimer {
     pt_ctx *ctx;
     bool on;
-    hipStream_t stream;
     uint64_t group;
     hipEvent_t a = nullptr;
-    EventTimer(pt_ctx *c, bool enabled, hipStream_t s = nullptr, uint64_t g = 0)
-        : ctx(c), on(enabled), stream(s ? s : c->stream), group(g ? g : (kGroupSingle | ++c->timer_groups)) {
+    EventTimer(pt_ctx *c, bool enabled, uint64_t g = 0)
+        : ctx(c), on(enabled), group(g ? g : (kGroupSingle | ++c->timer_groups)) {
         if (on) {
             a = next_event(ctx);
-            if (a) (void)hipEventRecord(a, stream);
+            if (a) (void)hipEventRecord(a, ctx->stream);
         }
     }
     // `also`: a second kind whose work the launch takes along (or -1).
@@ -1721,7 +1716,7 @@ struct EventTimer {
         if (!on || !a) return;
         hipEvent_t b = next_event(ctx);
         if (!b) return;
-        (void)hipEventRecord(b, stream);
+        (void)hipEventRecord(b, ctx->stream);
         ctx->pending.push_back(pt_ctx::Pending{kind, a, b, group});
         if (also >= 0) ctx->pending.push_back(pt_ctx::Pending{also, a, b, group});
     }
@@ -2411,7 +2406,7 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
     // bounce before it.
     const TraceKernel tk = trace_kernel(false, !b.spheres.empty());
     auto trace = [&](uint32_t bb) {
-        EventTimer t(ctx, timing, nullptr, launch_group ? (launch_group | (bb + 1)) : 0u);
+        EventTimer t(ctx, timing, launch_group ? (launch_group | (bb + 1)) : 0u);
         uint32_t *pair = counters + counter_pair(bb);
         const TraceJob job{ctx->q[bb & 1], pair, ctx->sq, bb ? pair + 1 : nullptr, ctx->d_out_l,
                            counters + counter_cursor(max_depth, bb), ctx->d_stat, b.d_roots, path_bits};
@@ -2429,17 +2424,17 @@ void batch_enqueue_launch(pt_ctx *ctx, const BatchShape &sh, uint32_t max_depth,
             GuideShadeArgs ga = bg.ga;
             ga.gout = infer_here ? ctx->d_gout : nullptr;
             if (infer_here) {
-                EventTimer t(ctx, timing, nullptr, group);
+                EventTimer t(ctx, timing, group);
                 launch_guide_infer(ctx, bg.view, in, count, path_bits, sv, sh.widest ? sh.widest : sh.capacity);
                 t.stop(kKindGuideInfer);
             }
-            EventTimer t(ctx, timing, nullptr, group);
+            EventTimer t(ctx, timing, group);
             hipLaunchKernelGGL(k_shade_guided<true>, dim3(sg), dim3(256), 0, ctx->stream, sv, sp, in, count, out,
                                counts_out, ctx->sq, ctx->d_out_l, aov, ga, (const BatchViewDev *)b.d_views, path_bits,
                                (const LaunchDesc *)b.d_launch);
             t.stop(kKindShade);
         } else {
-            EventTimer t(ctx, timing, nullptr, group);
+            EventTimer t(ctx, timing, group);
             hipLaunchKernelGGL(shade_kernel(true, b.feat), dim3(sg), dim3(sh.shade_block), 0, ctx->stream, sv, sp, in,
                                count, out, counts_out, ctx->sq, ctx->d_out_l, aov, (const BatchViewDev *)b.d_views,
                                path_bits);
@@ -3446,7 +3441,7 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
         // Timer groups: a bounce's kernels of one kind time as one launch.
         const uint64_t launch_group = (uint64_t)(batch + 1) << 16;
         {
-            EventTimer t(ctx, timing, nullptr, launch_group | 0xFFFFu);
+            EventTimer t(ctx, timing, launch_group | 0xFFFFu);
             const uint32_t grid = std::min<uint32_t>((total + 255) / 256, (uint32_t)ctx->num_cu * 32u);
             hipLaunchKernelGGL(k_raygen, dim3(grid), dim3(256), 0, ctx->stream, ctx->q[0], ctx->camera, ctx->width,
                                ctx->height, frames, seed, counters, ctx->num_counters);
@@ -3464,12 +3459,12 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
                 TraceJob sj = job;
                 sj.ext_count = nullptr;
                 sj.work = counters + counter_shadow_cursor(max_depth, b);
-                EventTimer t(ctx, timing, nullptr, launch_group | b);
+                EventTimer t(ctx, timing, launch_group | b);
                 hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, ctx->stream, sj, bvh);
                 t.stop(kKindShadow);
                 job.shd_count = nullptr;
             }
-            EventTimer t(ctx, timing, nullptr, launch_group | (b + 1));
+            EventTimer t(ctx, timing, launch_group | (b + 1));
             hipLaunchKernelGGL(tk, dim3(tg), dim3(kTraceBlock), 0, ctx->stream, job, bvh);
             t.stop(kKindTrace, job.shd_count ? kKindShadow : -1);
         };
@@ -3485,12 +3480,12 @@ static int pt_render_unguarded(pt_ctx *ctx, const pt_render_params *p) {
             GuideShadeArgs gac = ga;
             gac.gout = infer_here ? ctx->d_gout : nullptr;
             if (infer_here) {
-                EventTimer t(ctx, timing, nullptr, group);
+                EventTimer t(ctx, timing, group);
                 launch_guide_infer(ctx, gview, in, count, 31u, sv, total);
                 t.stop(kKindGuideInfer);
             }
             {
-                EventTimer t(ctx, timing, nullptr, group);
+                EventTimer t(ctx, timing, group);
                 if (guided)
                     hipLaunchKernelGGL(k_shade_guided<false>, dim3(sg), dim3(256), 0, ctx->stream, sv, sp, in, count, out,
                                        counts_out, ctx->sq, ctx->d_out_l, aov, gac, (const BatchViewDev *)nullptr, 31u,

@@ -143,18 +143,16 @@ def test_determinism(tracer):
 
 
 @pytest.mark.parametrize("guided", [False, True])
-def test_chained_launch_invariance(tracer, guided):
-    """A launch's paths run as up to four concurrent chains of kernels of at
-    least 10^6 paths (own queue parts, counters, streams and spill areas):
-    34 frames at 1920x1080 (one launch of four chains; then launches of 5
-    frames and one of 4, four chains each) and 3 single-frame launches (two
-    chains each) equal the same frames rendered with every launch as one
-    chain, bit for bit, AOVs and ray counts included; guided renders (network
-    inference, per-chain output buffers) too."""
+def test_shared_shadow_launch_invariance(tracer, guided):
+    """A traversal launch takes a bounce's extension rays and the shadow rays
+    of the bounce before; one_chain traces the shadow rays in launches of
+    their own.  Both render the same frames alike, bit for bit, AOVs and ray
+    counts included: 34 frames at 1920x1080 as one launch and as launches of 5
+    frames and one of 4, and 3 single-frame launches; guided renders (network
+    inference) too."""
     kind = pt.SCENE_DOOR_ROOM if guided else pt.SCENE_TERRAIN
-    print(f"case: {'door room' if guided else 'terrain'} 1920x1080, chained launches vs one chain", flush=True)
+    print(f"case: {'door room' if guided else 'terrain'} 1920x1080, shared vs separate shadow launches", flush=True)
     scene = pt.HostScene.generate(kind, seed=2)
-    assert scene.desc.width * scene.desc.height >= 2 * 10 ** 6  # a single 1080p frame splits into two chains
     tracer.set_scene(scene)
     tracer.build_bvh()
     kw = {"mis_mode": pt.MIS_CONSISTENT, "guide": True} if guided else {}

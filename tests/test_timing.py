@@ -1,8 +1,7 @@
 """Kernel active time (pupiloptixlab_amd/csrc/pt_timing.h): the union of a
-kernel kind's dispatch intervals, which the library reports per kernel kind
-when a launch's concurrent chains overlap, checked on the host by
-tests/timing_sim.cpp against a brute-force count on fixed and seeded random
-interval sets."""
+kernel kind's dispatch intervals, which the library reports per kernel kind,
+checked on the host by tests/timing_sim.cpp against a brute-force count on
+fixed and seeded random interval sets."""
 import os
 import subprocess
 
