@@ -523,9 +523,12 @@ struct GuideBins {
 };
 // Words of the cells; a launch's total sits after the blocks.
 constexpr size_t kBinWords = (2u << kBinBits) + kBinBlocks + 64u;
-// Queues of at least this many slots are sorted; at 58 K the three small
-// launches per bounce just pay for themselves (a training frame 4.75 -> 4.70
-// ms), below they would not.
+// Launches of at least this many paths are sorted, for three small launches a
+// bounce and 24 bytes per slot.  One guided frame of a closed room, in queue
+// order and sorted: 518 K paths 5.17 and 4.66 ms, 230 K 2.96 and 2.80, 100 K 2.03
+// and 1.94, 64 K 1.85 and 1.74.  The line lies where sorting just paid when a
+// launch ran as several chains; it pays below as well now (57 K 1.83 and 1.72 ms,
+// 15 K 1.72 and 1.63).
 constexpr uint32_t kBinMinPaths = 1u << 16;
 static_assert(kBinBlocks == 256, "k_guide_bin_move scans the blocks with its 256 threads");
 
@@ -1572,12 +1575,14 @@ uint32_t trace_grid(pt_ctx *ctx) {
 // them, at most kShadeRounds times the blocks that can be resident at once.
 // Every block strides over the queue; with many more blocks than slots the
 // dispatcher balances uneven shading work across CUs, and blocks that find no
-// work exit at once (terrain 1080p, 64 frames, image read back, at 1, 4, 16
-// and 64 rounds: 88.9, 87.2, 86.2 and 85.9 ms).  More blocks than slots only
-// cost their dispatch, 15 us a bounce (Cornell 320x180, one frame: 1.10 ->
-// 1.01 ms).  k_shade_guided<false> uses the same rounds when it only samples;
-// while training it keeps a grid of 8 blocks per CU (its training records are
-// indexed by path and vertex, so the grid does not change them).
+// work exit at once.  At 1, 4, 16 and 64 rounds, image read back: terrain 1080p,
+// 64 frames, 89.4, 87.0, 85.6 and 84.9 ms; textured terrain 771x433 4.96, 4.92,
+// 4.93 and 4.93; a closed room, whose paths cost alike, 18.1, 18.1, 18.2 and
+// 18.3, guided 35.4, 35.4, 35.6 and 35.5.  More blocks than slots only cost their
+// dispatch, 15 us a bounce (Cornell 320x180, one frame: 1.10 -> 1.01 ms).
+// k_shade_guided<false> uses the same rounds when it only samples; while
+// training it keeps a grid of 8 blocks per CU (its training records are indexed
+// by path and vertex, so the grid does not change them).
 uint32_t shade_grid(pt_ctx *ctx, bool guided, bool training, uint32_t paths) {
     const uint32_t need = (paths + 255u) / 256u, cus = (uint32_t)ctx->num_cu;
     if (guided && training) return std::min(need, cus * 8u);

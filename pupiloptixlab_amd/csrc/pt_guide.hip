@@ -1016,7 +1016,10 @@ bool GuideState::collect(const float4 *out_l, uint32_t total_paths, const GuideR
     }
     hipLaunchKernelGGL(k_guide_collect_begin, dim3(1), dim3(64), 0, stream, ctl);
     const uint32_t grid = std::max(1u, std::min<uint32_t>((r.capacity + 255) / 256, 4096u));
-    hipLaunchKernelGGL(k_guide_collect_count, dim3(std::min(grid, 2048u)), dim3(256), 0, stream, out_l, total_paths, r, ctl);
+    // The count takes as many blocks as are resident, each ends in two atomics on
+    // the same words (four 1080p training frames: 1.17 ms at 4096, 1.13 so).
+    hipLaunchKernelGGL(k_guide_collect_count, dim3(std::min(grid, 2048u)), dim3(256), 0, stream, out_l, total_paths, r,
+                       ctl);
     hipLaunchKernelGGL(k_guide_collect, dim3(grid), dim3(256), 0, stream, out_l, total_paths, r, samples, cap, ctl,
                        ring_n);
     if (ring_n)

@@ -1,7 +1,8 @@
 // Traversal of the compressed wide BVH by persistent waves that keep their
 // lanes busy: one ray per lane, and
 //   - a lane whose ray has ended takes the next one of the wave's share as soon
-//     as enough lanes are free, instead of waiting for the wave's slowest ray;
+//     as enough lanes are free, instead of waiting for the wave's slowest ray
+//     (dynamic ray fetch, Aila and Laine, HPG 2009);
 //   - leaf primitives are not tested where they are found.  The (lane,
 //     primitive) pairs of the wave's rays gather in a ring in LDS and are
 //     tested 64 at a time, one pair per lane, with the ray fetched from its
@@ -12,9 +13,10 @@
 //
 // Bound by VALU issue (97-100% busy alone).  With each wave walking 64 rays to
 // the end and testing leaves in place, an instruction had 20 of 64 lanes at
-// work on the terrain's rays and 30 in a closed room; now 43 and 45.  One
-// chain, 16 bounces: terrain, 33 M paths, 28.7 -> 21.8 ms; closed room, 8.3 M
-// paths, 19.7 -> 12.0 ms.
+// work on the terrain's rays and 30 in a closed room; now 43 and 45.  16
+// bounces, shadow rays in launches of their own: terrain, 33 M paths, 28.7 ->
+// 21.4 ms; closed room, 8.3 M paths, 19.7 -> 12.1 ms.  With them in the same
+// launches 18.7 and 11.6 ms, 45 lanes in both.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -52,11 +54,13 @@ __device__ __forceinline__ uint32_t from_lane(uint32_t v, uint32_t src) {
 // Free lanes that make the wave take new rays, and waiting rays (ended, pairs
 // untested) that make it test what is there: a refill costs the wave a ray's
 // set-up and its memory latency, a free lane its share of every instruction
-// (64 frames at 1080p: 88.7, 86.3 and 88.0 ms at 8, 16 and 24).
+// (8, 16 and 24: terrain 1080p, 64 frames, 86.5, 84.9 and 85.5 ms; closed room
+// 640x360, 32 frames, 18.9, 18.3 and 18.6 ms).
 constexpr uint32_t kRefillLanes = 16;
 // Pairs that make the wave test them: a partly filled test wastes lanes, a
-// late one lets its rays walk on past hits (88.0, 87.6, 87.0, 88.4 ms at 24,
-// 32, 48, 64 pairs).  With no more rays to take, as many as rays in flight.
+// late one lets its rays walk on past hits (24, 32, 40, 48 and 64: the same
+// terrain 86.2, 85.3, 84.9, 85.0 and 85.3 ms; the room 18.6, 18.4, 18.3, 18.3 and
+// 18.2 ms).  With no more rays to take, as many as rays in flight.
 constexpr uint32_t kFlushPairs = 40;
 
 // Traces `total` rays with all waves of the grid.  Wave `wave` starts with
