@@ -17,8 +17,8 @@ terrain variants at 1080p with per-view hash grids and a shared MLP; `--guided-b
 the 16 + 16 views).  The roofline block uses
 the kernel that takes longest alone (the traversal, which takes a bounce's
 extension rays together with the shadow rays of the bounce before); its algorithmic bytes come from a counting
-pass over the same frames (identical rays: the tracer is deterministic) and its
-time from HIP events recorded during the timed region (its active time: the
+pass over the same frames (the same rays, each walked by itself, so the counts are
+the same on every run) and its time from HIP events recorded during the timed region (its active time: the
 union of its dispatches' intervals); `roofline.single_chain` repeats the frames
 with shadow rays traced in launches of their own and prices the extension
 rays' kernel alone.  The CPU baseline is the oracle (scalar C++,
@@ -757,6 +757,9 @@ def main():
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
+            "priced": ("algorithmic bytes (rays, and the nodes and primitives that each ray's own walk visits) over the "
+                       "kernel's time; caches serve most of them, so frac is not a share of HBM's time and can pass 1: "
+                       "`limiter` says what bounds the kernel"),
             "traffic": traffic,
             "traffic_shape": None if traffic is None else
                              traffic_note or f"measured at this launch shape ({frames_per_launch} frames per launch)",
